@@ -3,12 +3,14 @@
 // weighted combine, all on the caller's stream, scratch from the caller's workspace.
 //
 // Data flow for T tokens, S slots per token (topk routed + the shared expert), R = T * S rows:
-//   router_kernel    logits[T, Er] = bf16(x @ router^T)                          (bf16 MFMA)
-//   route_kernel     ids[T, S], weights[T, S]: sigmoid, grouped top-k, shared slot last
-//   align_kernel     one workgroup: per-expert counts, the rows sorted by expert (stable only per
+//   router_kernel    fp32 partials over K ranges of x @ router^T                 (bf16 MFMA)
+//   route_kernel     logits[T, Er] = bf16(sum of the partials); ids[T, S], weights[T, S]: sigmoid, grouped
+//                    top-k, shared slot last
+//   align_quant_kernel, two halves side by side:
+//     sort           one workgroup: per-expert counts, the rows sorted by expert (stable only per
 //                    expert, which nothing depends on), each row's position, and the tables of
 //                    256-, 128- and 64-row blocks (expert, first row, rows) the GEMMs walk
-//   quant_div_kernel x -> e4m3 per 1 x 128 at scale max(amax / 448, tiny) (a true division, as the
+//     quantization   x -> e4m3 per 1 x 128 at scale max(amax / 448, tiny) (a true division, as the
 //                    checkpoint's FP8 scheme quantizes the linears' inputs), scales [D/128, T]
 //   moe_gemm<GATEUP> per block class, per (block, 128 columns of the intermediate): rows gathered by token, gate and up
 //                    weight rows interleaved per 16 so each lane holds both for the same columns;
@@ -40,138 +42,269 @@ constexpr float kFp32Tiny = 1.17549435e-38f;
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
 // ---------------------------------------------------------------------------------------------
-// router: one wave computes 16 tokens x 16 * NT experts with V_MFMA_F32_16X16X32_BF16, operands
-// straight from global memory: lane (li, g) loads the 8 bf16 at k0 + 8g of its row. The MFMA pairs
-// A's and B's lane groups the same way, so this assignment of k only has to match between them.
-template <int NT>
+// router: fp32 partial logits part[ks][T][E] of x @ router^T over K ranges, V_MFMA_F32_16X16X32_BF16 with
+// operands straight from global memory: lane (li, g) loads the 8 bf16 at k0 + 8g of its row. The MFMA
+// pairs A's and B's lane groups the same way, so this assignment of k only has to match between them.
+// A workgroup of 4 waves owns 16 * MT tokens x 16 * NT * (4 / KW) experts of one K range; with KW = 4 its
+// waves take a quarter of the range each and meet in LDS, in wave order. route_kernel adds the ranges.
+//
+// Bound by load latency: a wave that walks all of K in one chain of 224 load-to-MFMA round trips took
+// 94 us at 4 tokens x 256 experts x 7168 (3.7 MB), and 89 at 128. Splitting K over waves and workgroups
+// (plan_router) leaves each wave a few batches of UK steps, the next batch's loads in flight under the
+// current one's MFMAs: 4.9 us and 9.4.
+template <int MT, int NT, int KW, int UK>
 __global__ __launch_bounds__(256) void router_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ wr,
-                                                     uint16_t* __restrict__ logits, int T, int E, int D) {
+                                                     float* __restrict__ part, int T, int E, int D, int ks_count,
+                                                     int steps_per_wave) {
+  constexpr int EW = 4 / KW;
+  __shared__ f32x4 red[KW > 1 ? KW - 1 : 1][MT * NT][64];
   const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int tiles_e = (E + 16 * NT - 1) / (16 * NT);
-  const int tt = wave / tiles_e, te = wave % tiles_e;
-  if (tt * 16 >= T) return;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kw = KW > 1 ? w : 0, ew = KW > 1 ? 0 : w;
+  const int tiles_e = (E + 16 * NT * EW - 1) / (16 * NT * EW);
+  const int ks = blockIdx.x % ks_count, tile = blockIdx.x / ks_count;
+  const int t0 = (tile / tiles_e) * 16 * MT, e0 = ((tile % tiles_e) * EW + ew) * 16 * NT;
   const int li = lane & 15, g = lane >> 4;
-  const rsrc_t xr = make_rsrc(x + (int64_t)tt * 16 * D, (uint32_t)((int64_t)min(16, T - tt * 16) * D * 2));
-  const uint32_t x_off = li < T - tt * 16 ? (uint32_t)((li * D + 8 * g) * 2) : kOobOffset;
-  rsrc_t br[NT];
-  uint32_t b_off[NT];
+  const int s_begin = (ks * KW + kw) * steps_per_wave, s_end = min(D / 32, s_begin + steps_per_wave);
+  // rows past T and experts past E read the out-of-range offset (zeros)
+  const rsrc_t xr = make_rsrc(x + (int64_t)t0 * D, (uint32_t)((int64_t)min(16 * MT, T - t0) * D * 2));
+  const rsrc_t br = make_rsrc(wr + (int64_t)min(e0, E - 1) * D, (uint32_t)((int64_t)max(0, min(16 * NT, E - e0)) * D * 2));
+  uint32_t x_off[MT], b_off[NT];
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int e0 = te * 16 * NT + nt * 16;
-    br[nt] = make_rsrc(wr + (int64_t)min(e0, E - 1) * D, (uint32_t)((int64_t)max(0, min(16, E - e0)) * D * 2));
-    b_off[nt] = e0 + li < E ? (uint32_t)((li * D + 8 * g) * 2) : kOobOffset;
-  }
-  f32x4 acc[NT];
+  for (int mt = 0; mt < MT; ++mt)
+    x_off[mt] = t0 + mt * 16 + li < T ? (uint32_t)(((mt * 16 + li) * D + 8 * g) * 2) : kOobOffset;
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < D; k0 += 32) {
-    const uint32_t kb = (uint32_t)k0 * 2;
-    const bf16x8 a = __builtin_bit_cast(bf16x8, buf_ld16(xr, x_off + kb));
+  for (int nt = 0; nt < NT; ++nt)
+    b_off[nt] = e0 + nt * 16 + li < E ? (uint32_t)(((nt * 16 + li) * D + 8 * g) * 2) : kOobOffset;
+  f32x4 acc[MT][NT];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const bf16x8 b = __builtin_bit_cast(bf16x8, buf_ld16(br[nt], b_off[nt] + kb));
-      acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[nt], 0, 0, 0);
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 xa[2][UK][MT], xb[2][UK][NT];
+  auto load = [&](int buf, int s0) {
+#pragma unroll
+    for (int u = 0; u < UK; ++u) {
+      const bool on = s0 + u < s_end;
+      const uint32_t kb = (uint32_t)(s0 + u) * 64;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) xa[buf][u][mt] = buf_ld16(xr, on ? x_off[mt] + kb : kOobOffset);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) xb[buf][u][nt] = buf_ld16(br, on ? b_off[nt] + kb : kOobOffset);
     }
+  };
+  auto fma = [&](int buf) {
+#pragma unroll
+    for (int u = 0; u < UK; ++u)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xa[buf][u][mt]),
+                                                                __builtin_bit_cast(bf16x8, xb[buf][u][nt]),
+                                                                acc[mt][nt], 0, 0, 0);
+  };
+  load(0, s_begin);
+  for (int s0 = s_begin; s0 < s_end; s0 += 2 * UK) {
+    load(1, s0 + UK);
+    fma(0);
+    load(0, s0 + 2 * UK);
+    fma(1);
+  }
+  if constexpr (KW > 1) {
+    if (w > 0) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) red[w - 1][mt * NT + nt][lane] = acc[mt][nt];
+    }
+    __syncthreads();
+    if (w > 0) return;
+#pragma unroll
+    for (int v = 0; v < KW - 1; ++v)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] += red[v][mt * NT + nt][lane];
   }
   // lane holds tokens 4g + r, expert li of each tile
+  float* const out = part + (int64_t)ks * T * E;
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int e = te * 16 * NT + nt * 16 + li;
-    if (e >= E) continue;
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int t = tt * 16 + 4 * g + r;
-      if (t < T) logits[(int64_t)t * E + e] = (uint16_t)f32_to_bf16_bits(acc[nt][r]);
+    for (int nt = 0; nt < NT; ++nt) {
+      const int e = e0 + nt * 16 + li;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = t0 + mt * 16 + 4 * g + r;
+        if (t < T && e < E) out[(int64_t)t * E + e] = acc[mt][nt][r];
+      }
     }
-  }
+}
+
+// Router plan. One 16 x 16 tile a workgroup up to 16 tokens (all waves on K); 32 x 32 tiles, which halve the
+// operand reads per product, up to 1023 tokens or where the experts do not fill four waves; 64 x 256 tiles
+// (a wave per 64 experts) from 1024 tokens, where re-reading the weights per token tile is what counts.
+// K is cut until about 512 workgroups run, into at most 16 ranges (route_kernel reads one partial of each).
+struct RouterPlan {
+  int shape;  // 0: 16 x 16, 1: 32 x 32, 2: 64 x 256
+  int ranges, steps_per_wave;
+  int64_t groups;
+};
+
+static RouterPlan plan_router(int64_t T, int64_t E, int64_t D) {
+  RouterPlan p;
+  p.shape = T <= 16 ? 0 : ((T < 1024 || E <= 64) ? 1 : 2);
+  const int64_t tm = p.shape == 0 ? 16 : (p.shape == 1 ? 32 : 64), tn = p.shape == 0 ? 16 : (p.shape == 1 ? 32 : 256);
+  const int64_t tiles = ((T + tm - 1) / tm) * ((E + tn - 1) / tn);
+  const int64_t waves = p.shape == 2 ? 1 : 4, steps = D / 32;
+  int64_t r = 512 / tiles;
+  r = r < 1 ? 1 : (r > 16 ? 16 : r);
+  p.steps_per_wave = (int)((steps + r * waves - 1) / (r * waves));
+  p.ranges = (int)((steps + p.steps_per_wave * waves - 1) / (p.steps_per_wave * waves));
+  p.groups = tiles * p.ranges;
+  return p;
 }
 
 // ---------------------------------------------------------------------------------------------
-// route: one wave per token. (value, index) pairs compare by value, then the lower index first.
-__device__ __forceinline__ bool better(float v, int i, float w, int j) { return v > w || (v == w && i < j); }
+// route: one wave per token. (value, index) pairs compare by value, then the lower index first; a NaN is
+// never picked. As one 64-bit key: the value's bits in an unsigned order, then the inverted index; 0 marks
+// no candidate. The wave's maximum takes four DPP moves and two lane swaps, no LDS permutes (with 12
+// maxima a token in 12 permutes each, the kernel took 15.5 us at 4 tokens of 256 experts in 8 groups and 47
+// at 4096 ungrouped; now 6.9, the router's partials included, and 10.2).
+constexpr int kNoIndex = 1 << 30;
 
-__device__ __forceinline__ void wave_argmax(float& v, int& i) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const float w = __shfl_xor(v, off);
-    const int j = __shfl_xor(i, off);
-    if (better(w, j, v, i)) {
-      v = w;
-      i = j;
-    }
-  }
+__device__ __forceinline__ uint64_t rank_key(float v, int i) {
+  if (!(v == v)) return 0;
+  const uint32_t u = __float_as_uint(v + 0.0f);  // -0 counts as 0
+  return ((uint64_t)(u ^ ((u & 0x80000000u) ? 0xFFFFFFFFu : 0x80000000u)) << 32) | (uint32_t)~i;
+}
+__device__ __forceinline__ int key_index(uint64_t k) { return k == 0 ? kNoIndex : (int)~(uint32_t)k; }
+
+template <int CTRL>
+__device__ __forceinline__ uint64_t dpp_max(uint64_t k) {
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)k, CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(k >> 32), CTRL, 0xF, 0xF, false);
+  const uint64_t o = ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo;
+  return o > k ? o : k;
 }
 
-constexpr int kRouteMaxPerLane = 16;  // routed experts <= 1024
+__device__ __forceinline__ uint64_t wave_max(uint64_t k) {
+  k = dpp_max<0xB1>(k);   // quad_perm [1,0,3,2]
+  k = dpp_max<0x4E>(k);   // quad_perm [2,3,0,1]
+  k = dpp_max<0x141>(k);  // row_half_mirror: the other quad of the 8
+  k = dpp_max<0x140>(k);  // row_mirror: the other 8 of the 16
+  {
+    const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)k, (uint32_t)k, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(k >> 32), (uint32_t)(k >> 32), false, false);
+    const uint64_t a = ((uint64_t)hi[0] << 32) | lo[0], b = ((uint64_t)hi[1] << 32) | lo[1];
+    k = a > b ? a : b;
+  }
+  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)k, (uint32_t)k, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(k >> 32), (uint32_t)(k >> 32), false, false);
+  const uint64_t a = ((uint64_t)hi[0] << 32) | lo[0], b = ((uint64_t)hi[1] << 32) | lo[1];
+  return a > b ? a : b;
+}
 
-__global__ __launch_bounds__(64) void route_kernel(const uint16_t* __restrict__ logits, const uint16_t* __restrict__ bias,
-                                                   int T, int E, int G, int topk, int topk_group, int renormalize,
-                                                   float scale, int shared, int32_t* __restrict__ ids,
-                                                   float* __restrict__ weights) {
-  __shared__ float sv[1024];  // unbiased scores
-  __shared__ float sb[1024];  // biased scores
+// Logits: bf16 [T, E], or fp32 partials [ranges][T, E] whose sum, in range order, is rounded to bf16.
+// PER_LANE * 64 experts at most (4: up to 256, 16: up to 1024); lane l holds experts l, l + 64, ...
+template <bool PART, int PER_LANE>
+__global__ __launch_bounds__(64) void route_kernel(const uint16_t* __restrict__ logits, const float* __restrict__ part,
+                                                   int ranges, const uint16_t* __restrict__ bias, int T, int E, int G,
+                                                   int topk, int topk_group, int renormalize, float scale, int shared,
+                                                   int32_t* __restrict__ ids, float* __restrict__ weights) {
+  __shared__ float sv[64 * PER_LANE];  // unbiased scores
+  __shared__ float sb[64 * PER_LANE];  // biased scores
   const int t = blockIdx.x;
   const int lane = threadIdx.x;
   const int per = E / G;
-  float b[kRouteMaxPerLane];
+  float x[PER_LANE], bs[PER_LANE];
 #pragma unroll
-  for (int j = 0; j < kRouteMaxPerLane; ++j) {
+  for (int j = 0; j < PER_LANE; ++j) {
+    const int i = min(lane + 64 * j, E - 1);
+    x[j] = PART ? part[(int64_t)t * E + i] : bf16_to_f32(logits[(int64_t)t * E + i]);
+    bs[j] = bf16_to_f32(bias[i]);
+  }
+  if constexpr (PART) {
+    // the partials come from other XCDs' writes, a long way off: kRouteBatch ranges' loads at a time
+    constexpr int kRouteBatch = PER_LANE == 4 ? 15 : 5;
+    for (int k0 = 1; k0 < ranges; k0 += kRouteBatch) {
+      float v[kRouteBatch][PER_LANE];
+#pragma unroll
+      for (int k = 0; k < kRouteBatch; ++k)
+#pragma unroll
+        for (int j = 0; j < PER_LANE; ++j)
+          v[k][j] = part[((int64_t)min(k0 + k, ranges - 1) * T + t) * E + min(lane + 64 * j, E - 1)];
+#pragma unroll
+      for (int k = 0; k < kRouteBatch; ++k)
+#pragma unroll
+        for (int j = 0; j < PER_LANE; ++j) x[j] += k0 + k < ranges ? v[k][j] : 0.0f;
+    }
+  }
+  uint64_t key[PER_LANE];
+#pragma unroll
+  for (int j = 0; j < PER_LANE; ++j) {
     const int i = lane + 64 * j;
-    b[j] = -INFINITY;
+    key[j] = 0;
     if (i < E) {
-      const float x = bf16_to_f32(logits[(int64_t)t * E + i]);
-      const float v = 1.0f / (1.0f + expf(-x));
-      b[j] = v + bf16_to_f32(bias[i]);
+      const float lx = PART ? __uint_as_float(f32_to_bf16_bits(x[j]) << 16) : x[j];
+      const float v = 1.0f / (1.0f + expf(-lx));
+      const float b = v + bs[j];
+      key[j] = rank_key(b, i);
       sv[i] = v;
-      sb[i] = b[j];
+      sb[i] = b;
     }
   }
   __syncthreads();
-  // group score: the sum of its two best biased scores
-  float gs = -INFINITY;
-  if (lane < G) {
+  uint64_t kept = ~0ull;
+  if (G > 1 || topk_group != 1) {
+    // group score: the sum of its two best biased scores, found by nsub lanes a group (a power of two)
+    int nsub = 64;
+    while (nsub * G > 64) nsub >>= 1;
+    const int gi = lane / nsub, sub = lane % nsub;
     float m1 = -INFINITY, m2 = -INFINITY;
-    for (int i = lane * per; i < lane * per + per; ++i) {
-      const float x = sb[i];
-      if (x > m1) {
-        m2 = m1;
-        m1 = x;
-      } else if (x > m2) {
-        m2 = x;
+    if (gi < G)
+      for (int i = gi * per + sub; i < gi * per + per; i += nsub) {
+        const float v = sb[i];
+        if (v > m1) {
+          m2 = m1;
+          m1 = v;
+        } else if (v > m2) {
+          m2 = v;
+        }
       }
+    for (int off = nsub >> 1; off >= 1; off >>= 1) {
+      const float o1 = __shfl_xor(m1, off), o2 = __shfl_xor(m2, off);
+      m2 = fmaxf(fminf(m1, o1), fmaxf(m2, o2));
+      m1 = fmaxf(m1, o1);
     }
-    gs = m1 + m2;
-  }
-  // keep the topk_group best groups (G <= 64)
-  uint64_t kept = 0;
-  bool mine = false;
-  for (int r = 0; r < topk_group; ++r) {
-    float v = (lane < G && !mine) ? gs : -INFINITY;
-    int i = lane < G && !mine ? lane : 1 << 30;
-    wave_argmax(v, i);
-    if (i == lane) mine = true;
-    kept |= 1ull << (i & 63);
+    // keep the topk_group best groups (G <= 64); sub-lane 0 speaks for its group
+    uint64_t gk = (gi < G && sub == 0) ? rank_key(m1 + m2, gi) : 0;
+    kept = 0;
+    for (int r = 0; r < topk_group; ++r) {
+      const int i = key_index(wave_max(gk));
+      if (gk != 0 && i == gi) gk = 0;
+      kept |= 1ull << (i & 63);
+    }
+#pragma unroll
+    for (int j = 0; j < PER_LANE; ++j) {
+      const int e = min(lane + 64 * j, E - 1);
+      if (!(kept >> (e / per) & 1ull)) key[j] = 0;
+    }
   }
   // the topk best biased scores among the kept groups' experts
-  uint32_t taken = 0;
   float wsum = 0.0f;
   int my_id = 0;
   float my_v = 0.0f;
   for (int r = 0; r < topk; ++r) {
-    float v = -INFINITY;
-    int i = 1 << 30;
+    uint64_t best = key[0];
 #pragma unroll
-    for (int j = 0; j < kRouteMaxPerLane; ++j) {
-      const int e = lane + 64 * j;
-      if (e < E && !(taken >> j & 1u) && (kept >> (e / per) & 1ull) && better(b[j], e, v, i)) {
-        v = b[j];
-        i = e;
-      }
-    }
-    wave_argmax(v, i);
-    if ((i & 63) == lane) taken |= 1u << (i >> 6);
-    const float sc = sv[i];
+    for (int j = 1; j < PER_LANE; ++j) best = key[j] > best ? key[j] : best;
+    best = wave_max(best);
+#pragma unroll
+    for (int j = 0; j < PER_LANE; ++j) key[j] = key[j] == best ? 0 : key[j];
+    const int i = key_index(best);
+    const float sc = i == kNoIndex ? 0.0f : sv[i];
     wsum += sc;
     if (lane == r) {
       my_id = i;
@@ -191,7 +324,7 @@ __global__ __launch_bounds__(64) void route_kernel(const uint16_t* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------------------------
-// align: one 1024-thread workgroup. Entries whose expert is out of [0, E) get row -1 (ignored).
+// align (the sort): one 1024-thread workgroup. Entries whose expert is out of [0, E) get row -1 (ignored).
 __device__ int block_exclusive_scan(int v, int* wsum, int* total) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   int incl = v;
@@ -233,53 +366,77 @@ __device__ __forceinline__ int class_blocks(int c, int k) {
   return (k == 0 ? full : 0) + (k == last ? 1 : 0);
 }
 
-__global__ __launch_bounds__(1024) void align_kernel(const int32_t* __restrict__ ids, int R, int S, int E,
-                                                     int32_t* __restrict__ row_of, int32_t* __restrict__ sorted_tok,
-                                                     BlockTable bt, int* __restrict__ tickets) {
-  __shared__ int cnt[kMaxExperts];
-  __shared__ int off[kMaxExperts];
-  __shared__ int boff[kClasses][kMaxExperts];
-  __shared__ int wsum[16];
-  __shared__ int total;
+struct AlignSmem {
+  int cnt[kMaxExperts];
+  int off[kMaxExperts];
+  int boff[kClasses][kMaxExperts];
+  int wsum[16];
+  int total;
+};
+
+// kAlignBatch ids a thread are loaded before the first is used: the two walks over the R slots are chains
+// of load, LDS atomic and store, and one id at a time they took 54 us at 36864 slots (46 now, with the
+// quantization of 4096 rows in the same launch).
+constexpr int kAlignBatch = 8;
+
+__device__ void align_block(AlignSmem& sm, const int32_t* __restrict__ ids, int R, int S, int E,
+                            int32_t* __restrict__ row_of, int32_t* __restrict__ sorted_tok, const BlockTable& bt,
+                            int* __restrict__ tickets) {
   const int tid = threadIdx.x;
   if (tid < 2) tickets[tid] = 0;  // the grouped GEMMs' work-item counters (gate-up, down)
-  for (int e = tid; e < kMaxExperts; e += 1024) cnt[e] = 0;
+  for (int e = tid; e < kMaxExperts; e += 1024) sm.cnt[e] = 0;
   __syncthreads();
-  for (int i = tid; i < R; i += 1024) {
-    const int e = ids[i];
-    row_of[i] = (e >= 0 && e < E) ? atomicAdd(&cnt[e], 1) : -1;
+  for (int i0 = tid; i0 < R; i0 += 1024 * kAlignBatch) {
+    int e[kAlignBatch], r[kAlignBatch];
+#pragma unroll
+    for (int j = 0; j < kAlignBatch; ++j) e[j] = i0 + 1024 * j < R ? ids[i0 + 1024 * j] : -1;
+#pragma unroll
+    for (int j = 0; j < kAlignBatch; ++j) r[j] = (e[j] >= 0 && e[j] < E) ? atomicAdd(&sm.cnt[e[j]], 1) : -1;
+#pragma unroll
+    for (int j = 0; j < kAlignBatch; ++j)
+      if (i0 + 1024 * j < R) row_of[i0 + 1024 * j] = r[j];
   }
   __syncthreads();
   // two experts per thread: exclusive prefix of rows, then of each class's blocks
   const int e0 = 2 * tid, e1 = 2 * tid + 1;
-  const int c0 = e0 < E ? cnt[e0] : 0, c1 = e1 < E ? cnt[e1] : 0;
-  const int o = block_exclusive_scan(c0 + c1, wsum, &total);
-  if (e0 < kMaxExperts) off[e0] = o;
-  if (e1 < kMaxExperts) off[e1] = o + c0;
+  const int c0 = e0 < E ? sm.cnt[e0] : 0, c1 = e1 < E ? sm.cnt[e1] : 0;
+  const int o = block_exclusive_scan(c0 + c1, sm.wsum, &sm.total);
+  if (e0 < kMaxExperts) sm.off[e0] = o;
+  if (e1 < kMaxExperts) sm.off[e1] = o + c0;
 #pragma unroll
   for (int k = 0; k < kClasses; ++k) {
     const int b0 = class_blocks(c0, k), b1 = class_blocks(c1, k);
-    const int bo = block_exclusive_scan(b0 + b1, wsum, &total);
-    if (e0 < kMaxExperts) boff[k][e0] = bo;
-    if (e1 < kMaxExperts) boff[k][e1] = bo + b0;
-    if (tid == 0) bt.count[k] = total;
+    const int bo = block_exclusive_scan(b0 + b1, sm.wsum, &sm.total);
+    if (e0 < kMaxExperts) sm.boff[k][e0] = bo;
+    if (e1 < kMaxExperts) sm.boff[k][e1] = bo + b0;
+    if (tid == 0) bt.count[k] = sm.total;
   }
   __syncthreads();
-  for (int i = tid; i < R; i += 1024) {
-    const int e = ids[i];
-    if (e < 0 || e >= E) continue;
-    const int pos = off[e] + row_of[i];
-    row_of[i] = pos;
-    sorted_tok[pos] = i / S;
+  for (int i0 = tid; i0 < R; i0 += 1024 * kAlignBatch) {
+    int e[kAlignBatch], r[kAlignBatch];
+#pragma unroll
+    for (int j = 0; j < kAlignBatch; ++j) {
+      const int i = i0 + 1024 * j;
+      e[j] = i < R ? ids[i] : -1;
+      r[j] = i < R ? row_of[i] : -1;  // this thread's own store
+    }
+#pragma unroll
+    for (int j = 0; j < kAlignBatch; ++j) {
+      const int i = i0 + 1024 * j;
+      if (e[j] < 0 || e[j] >= E) continue;
+      const int pos = sm.off[e[j]] + r[j];
+      row_of[i] = pos;
+      sorted_tok[pos] = i / S;
+    }
   }
   for (int e = tid; e < E; e += 1024) {
-    const int c = cnt[e];
-    int row = off[e], left = c;
+    const int c = sm.cnt[e];
+    int row = sm.off[e], left = c;
 #pragma unroll
     for (int k = 0; k < kClasses; ++k) {
       const int nb = class_blocks(c, k);
       for (int j = 0; j < nb; ++j) {
-        const int idx = k * bt.cap + boff[k][e] + j;
+        const int idx = k * bt.cap + sm.boff[k][e] + j;
         const int n = min(class_rows(k), left);
         bt.expert[idx] = e;
         bt.row[idx] = row;
@@ -291,13 +448,12 @@ __global__ __launch_bounds__(1024) void align_kernel(const int32_t* __restrict__
   }
 }
 
-// ---------------------------------------------------------------------------------------------
 // quant: 16 lanes per 1 x 128 group, 8 values each. scale = max(amax / 448, tiny); code =
 // e4m3(x / scale), both true IEEE divisions.
-__global__ __launch_bounds__(256) void quant_div_kernel(const uint16_t* __restrict__ x, int T, int D,
-                                                        uint8_t* __restrict__ q, float* __restrict__ s) {
+__device__ void quant_div_block(int block, const uint16_t* __restrict__ x, int T, int D, uint8_t* __restrict__ q,
+                                float* __restrict__ s) {
   const int groups = D / 128;
-  const int gid = blockIdx.x * 16 + (threadIdx.x >> 4);
+  const int gid = block * 64 + (threadIdx.x >> 4);
   if (gid >= T * groups) return;
   const int t = gid / groups, grp = gid - t * groups;
   const int sub = threadIdx.x & 15;
@@ -312,8 +468,10 @@ __global__ __launch_bounds__(256) void quant_div_kernel(const uint16_t* __restri
   float amax = 0.0f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(f[i]));
-#pragma unroll
-  for (int off = 1; off < 16; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+  amax = fmaxf(amax, dpp_f32<0xB1>(amax));   // the group's 16 lanes are one DPP row: quad_perm [1,0,3,2]
+  amax = fmaxf(amax, dpp_f32<0x4E>(amax));   // quad_perm [2,3,0,1]
+  amax = fmaxf(amax, dpp_f32<0x141>(amax));  // row_half_mirror
+  amax = fmaxf(amax, dpp_f32<0x140>(amax));  // row_mirror
   const float sc = fmaxf(__fdiv_rn(amax, 448.0f), kFp32Tiny);
   float c[8];
 #pragma unroll
@@ -323,6 +481,22 @@ __global__ __launch_bounds__(256) void quant_div_kernel(const uint16_t* __restri
   out[1] = pack4_e4m3(c[4], c[5], c[6], c[7]);
   *reinterpret_cast<u32x2*>(q + base) = out;
   if (sub == 0) s[(int64_t)grp * T + t] = sc;
+}
+
+// One launch for the expert sort (workgroup 0) and the input quantization (the others): neither needs the
+// other, so the sort's single workgroup runs beside the quantization instead of before it (5.4 + 5.2 us
+// apart at 4 tokens, 53.8 + 26.0 at 4096; 6.3 and 45.9 together).
+__global__ __launch_bounds__(1024) void align_quant_kernel(const int32_t* __restrict__ ids, int R, int S, int E,
+                                                           int32_t* __restrict__ row_of,
+                                                           int32_t* __restrict__ sorted_tok, BlockTable bt,
+                                                           int* __restrict__ tickets, const uint16_t* __restrict__ x,
+                                                           int T, int D, uint8_t* __restrict__ q,
+                                                           float* __restrict__ s) {
+  __shared__ AlignSmem sm;
+  if (blockIdx.x == 0)
+    align_block(sm, ids, R, S, E, row_of, sorted_tok, bt, tickets);
+  else
+    quant_div_block((int)blockIdx.x - 1, x, T, D, q, s);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -343,7 +517,7 @@ struct MoeGemmArgs {
   const int32_t* blk_rows;
   const int32_t* nblk;        // blocks per class
   int blk_cap;
-  int* tickets;               // work-item counter, zero at launch (align_kernel clears it)
+  int* tickets;               // work-item counter, zero at launch (align_block clears it)
   int K, N, I;               // reduction length, weight rows, intermediate size
   int tiles_n;               // GATEUP: I / 128; DOWN: ceil(N / 256)
   uint8_t* hq;               // GATEUP out: [R, I] codes
@@ -669,35 +843,51 @@ __global__ __launch_bounds__(512) void moe_gemm_kernel(MoeGemmArgs p) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// combine: out[t] = bf16(sum over slots in slot order of weight * y[row]); 8 columns per thread.
-__global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict__ y, const int32_t* __restrict__ row_of,
-                                                      const float* __restrict__ weights, int S, int D,
-                                                      uint16_t* __restrict__ out) {
+// combine: out[t] = bf16(sum over slots in slot order of weight * y[row]); 8 columns per thread. The rows
+// of kCombineBatch slots load together: one row at a time (an index load, then the row it names) the
+// kernel took 15.6 us at 4 tokens x 9 slots of 7168, whose bytes take a microsecond; together 4.8. At 4096
+// tokens the rows' 590 MB bound it (119.7 -> 117.6 us).
+constexpr int kCombineBatch = 9, kCombineThreads = 128;
+__global__ __launch_bounds__(kCombineThreads) void combine_kernel(const uint16_t* __restrict__ y,
+                                                                  const int32_t* __restrict__ row_of,
+                                                                  const float* __restrict__ weights, int S, int D,
+                                                                  uint16_t* __restrict__ out) {
   const int t = blockIdx.x;
-  for (int c0 = threadIdx.x * 8; c0 < D; c0 += 256 * 8) {
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < S; ++s) {
-      const int row = row_of[(int64_t)t * S + s];
-      if (row < 0) continue;
-      const float wt = weights[(int64_t)t * S + s];
-      const u32x4 v = ld16(y + (int64_t)row * D + c0);
+  const int c0 = (blockIdx.y * kCombineThreads + threadIdx.x) * 8;
+  if (c0 >= D) return;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < S; s0 += kCombineBatch) {
+    int row[kCombineBatch];
+    float wt[kCombineBatch];
+    u32x4 v[kCombineBatch];
+#pragma unroll
+    for (int j = 0; j < kCombineBatch; ++j) {
+      const int64_t i = (int64_t)t * S + min(s0 + j, S - 1);
+      row[j] = s0 + j < S ? row_of[i] : -1;
+      wt[j] = weights[i];
+    }
+#pragma unroll
+    for (int j = 0; j < kCombineBatch; ++j) v[j] = ld16(y + (int64_t)max(row[j], 0) * D + c0);
+#pragma unroll
+    for (int j = 0; j < kCombineBatch; ++j) {
+      if (row[j] < 0) continue;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        acc[2 * i] = fmaf(wt, bf16_lo(v[i]), acc[2 * i]);
-        acc[2 * i + 1] = fmaf(wt, bf16_hi(v[i]), acc[2 * i + 1]);
+        acc[2 * i] = fmaf(wt[j], bf16_lo(v[j][i]), acc[2 * i]);
+        acc[2 * i + 1] = fmaf(wt[j], bf16_hi(v[j][i]), acc[2 * i + 1]);
       }
     }
-    u32x4 o;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = pack_bf16x2(acc[2 * i], acc[2 * i + 1]);
-    *reinterpret_cast<u32x4*>(out + (int64_t)t * D + c0) = o;
   }
+  u32x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o[i] = pack_bf16x2(acc[2 * i], acc[2 * i + 1]);
+  *reinterpret_cast<u32x4*>(out + (int64_t)t * D + c0) = o;
 }
 
 // ---------------------------------------------------------------------------------------------
 // host side
 struct Workspace {
-  size_t logits, ids, weights, row_of, sorted_tok, blk_expert, blk_row, blk_rows, nblk, tickets, xq, xs, hq, hs, y,
+  size_t part, ids, weights, row_of, sorted_tok, blk_expert, blk_row, blk_rows, nblk, tickets, xq, xs, hq, hs, y,
       total;
   int blk_cap;  // block-table entries per class
 };
@@ -718,7 +908,7 @@ static Workspace layout(int64_t T, int64_t S, int64_t D, int64_t I, int64_t E, i
     o = align256(o + bytes);
     return at;
   };
-  w.logits = take((size_t)(T * Er * 2));
+  w.part = take(Er ? (size_t)(plan_router(T, Er, D).ranges * T * Er * 4) : 0);
   w.ids = take((size_t)(Er ? R * 4 : 0));
   w.weights = take((size_t)(Er ? R * 4 : 0));
   w.row_of = take((size_t)R * 4);
@@ -761,6 +951,28 @@ static void launch_gemms(const MoeGemmArgs& gu, const MoeGemmArgs& dn, hipStream
   hipLaunchKernelGGL((moe_gemm_kernel<kDown, PRE>), grid, dim3(512), 0, stream, dn);
 }
 
+// Grouped top-k on bf16 logits, or (part) on the router's fp32 partials.
+static void launch_route(const uint16_t* logits, const float* part, int ranges, const uint16_t* bias, int64_t T,
+                         int64_t E, int G, int topk, int topk_group, int renormalize, float scale, int shared,
+                         int32_t* ids, float* weights, hipStream_t stream) {
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)T), dim3(64), 0, stream, logits, part, ranges, bias, (int)T, (int)E, G,
+                       topk, topk_group, renormalize ? 1 : 0, scale, shared ? 1 : 0, ids, weights);
+  };
+  if (part)
+    E <= 256 ? go(route_kernel<true, 4>) : go(route_kernel<true, 16>);
+  else
+    E <= 256 ? go(route_kernel<false, 4>) : go(route_kernel<false, 16>);
+}
+
+// The arguments the grouped top-k takes.
+static bool route_ok(int64_t tokens, int64_t n_routed, int topk, int num_expert_group, int topk_group) {
+  if (tokens <= 0 || tokens > 65536 || n_routed < 2 || n_routed > 1024) return false;
+  if (num_expert_group < 1 || num_expert_group > 64 || n_routed % num_expert_group) return false;
+  if (n_routed / num_expert_group < 2 || topk_group < 1 || topk_group > num_expert_group) return false;
+  return topk >= 1 && topk <= 63 && topk <= topk_group * (n_routed / num_expert_group);
+}
+
 // Experts on a routing already in ids/weights ([T, S], slots in [0, E); others are skipped).
 static int run_experts(const uint16_t* hidden, int64_t T, int64_t D, int64_t I, int64_t E, const int32_t* ids,
                        const float* weights, int64_t S, const uint8_t* w1, const float* w1s, const uint8_t* w2,
@@ -782,11 +994,9 @@ static int run_experts(const uint16_t* hidden, int64_t T, int64_t D, int64_t I, 
   uint16_t* y = reinterpret_cast<uint16_t*>(ws + L.y);
   int* tickets = reinterpret_cast<int*>(ws + L.tickets);
 
-  hipLaunchKernelGGL(align_kernel, dim3(1), dim3(1024), 0, stream, ids, (int)R, (int)S, (int)E, row_of, sorted_tok, bt,
-                     tickets);
   const int64_t qgroups = T * (D / 128);
-  hipLaunchKernelGGL(quant_div_kernel, dim3((unsigned)((qgroups + 15) / 16)), dim3(256), 0, stream, hidden, (int)T,
-                     (int)D, xq, xs);
+  hipLaunchKernelGGL(align_quant_kernel, dim3((unsigned)(1 + (qgroups + 63) / 64)), dim3(1024), 0, stream, ids, (int)R,
+                     (int)S, (int)E, row_of, sorted_tok, bt, tickets, hidden, (int)T, (int)D, xq, xs);
   MoeGemmArgs gu{};
   gu.a = xq;
   gu.sa = xs;
@@ -827,7 +1037,8 @@ static int run_experts(const uint16_t* hidden, int64_t T, int64_t D, int64_t I, 
     launch_gemms<true>(gu, dn, stream);
   else
     launch_gemms<false>(gu, dn, stream);
-  hipLaunchKernelGGL(combine_kernel, dim3((unsigned)T), dim3(256), 0, stream, y, row_of, weights, (int)S, (int)D, out);
+  hipLaunchKernelGGL(combine_kernel, dim3((unsigned)T, (unsigned)((D / 8 + kCombineThreads - 1) / kCombineThreads)),
+                     dim3(kCombineThreads), 0, stream, y, row_of, weights, (int)S, (int)D, out);
   AKLR_LAUNCH_CHECK();
   return AKLR_OK;
 }
@@ -848,13 +1059,10 @@ extern "C" int aklr_moe_fp8_route(const void* logits, const void* bias, int64_t 
                                   int num_expert_group, int topk_group, int renormalize, float routed_scaling_factor,
                                   int append_shared, int32_t* ids, float* weights, hipStream_t stream) {
   if (!logits || !bias || !ids || !weights) return AKLR_ERR_INVALID_ARGUMENT;
-  if (tokens <= 0 || tokens > 65536 || n_routed < 2 || n_routed > 1024) return AKLR_ERR_INVALID_ARGUMENT;
-  if (num_expert_group < 1 || num_expert_group > 64 || n_routed % num_expert_group) return AKLR_ERR_INVALID_ARGUMENT;
-  if (n_routed / num_expert_group < 2 || topk_group < 1 || topk_group > num_expert_group) return AKLR_ERR_INVALID_ARGUMENT;
-  if (topk < 1 || topk > 63 || topk > topk_group * (n_routed / num_expert_group)) return AKLR_ERR_INVALID_ARGUMENT;
-  hipLaunchKernelGGL(route_kernel, dim3((unsigned)tokens), dim3(64), 0, stream, static_cast<const uint16_t*>(logits),
-                     static_cast<const uint16_t*>(bias), (int)tokens, (int)n_routed, num_expert_group, topk, topk_group,
-                     renormalize ? 1 : 0, routed_scaling_factor, append_shared ? 1 : 0, ids, weights);
+  if (!route_ok(tokens, n_routed, topk, num_expert_group, topk_group)) return AKLR_ERR_INVALID_ARGUMENT;
+  launch_route(static_cast<const uint16_t*>(logits), nullptr, 0, static_cast<const uint16_t*>(bias), tokens, n_routed,
+               num_expert_group, topk, topk_group, renormalize, routed_scaling_factor, append_shared, ids, weights,
+               stream);
   AKLR_LAUNCH_CHECK();
   return AKLR_OK;
 }
@@ -884,7 +1092,7 @@ extern "C" int aklr_deepseek_v2_fp8_moe(const void* hidden, const void* router_w
                                         size_t workspace_bytes, hipStream_t stream) {
   if (!hidden || !router_weight || !correction_bias || !w1 || !w1_scale || !w2 || !w2_scale || !out)
     return AKLR_ERR_INVALID_ARGUMENT;
-  if (n_routed < 2 || n_routed > 1024 || topk < 1 || topk > 63) return AKLR_ERR_INVALID_ARGUMENT;
+  if (!route_ok(tokens, n_routed, topk, num_expert_group, topk_group)) return AKLR_ERR_INVALID_ARGUMENT;
   const int64_t S = topk + 1, E = n_routed + 1;
   if (!dims_ok(tokens, model_dim, inter_dim, E, S)) return AKLR_ERR_INVALID_ARGUMENT;
   if (w_layout != AKLR_B_ROW_MAJOR && w_layout != AKLR_B_PRESHUFFLE_16x16) return AKLR_ERR_UNSUPPORTED;
@@ -894,22 +1102,23 @@ extern "C" int aklr_deepseek_v2_fp8_moe(const void* hidden, const void* router_w
   const Workspace L = layout(tokens, S, model_dim, inter_dim, E, n_routed);
   if (!workspace || workspace_bytes < L.total || !aklr_aligned16(workspace)) return AKLR_ERR_WORKSPACE;
   uint8_t* ws = static_cast<uint8_t*>(workspace);
-  uint16_t* logits = reinterpret_cast<uint16_t*>(ws + L.logits);
+  float* part = reinterpret_cast<float*>(ws + L.part);
   int32_t* ids = reinterpret_cast<int32_t*>(ws + L.ids);
   float* weights = reinterpret_cast<float*>(ws + L.weights);
-  const int nt = tokens >= 1024 ? 4 : 1;
-  const int64_t waves = ((tokens + 15) / 16) * ((n_routed + 16 * nt - 1) / (16 * nt));
-  if (nt == 4)
-    hipLaunchKernelGGL((router_kernel<4>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream,
-                       static_cast<const uint16_t*>(hidden), static_cast<const uint16_t*>(router_weight), logits,
-                       (int)tokens, (int)n_routed, (int)model_dim);
+  const RouterPlan rp = plan_router(tokens, n_routed, model_dim);
+  const auto router = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)rp.groups), dim3(256), 0, stream, static_cast<const uint16_t*>(hidden),
+                       static_cast<const uint16_t*>(router_weight), part, (int)tokens, (int)n_routed, (int)model_dim,
+                       rp.ranges, rp.steps_per_wave);
+  };
+  if (rp.shape == 0)
+    router(router_kernel<1, 1, 4, 4>);
+  else if (rp.shape == 1)
+    router(router_kernel<2, 2, 4, 4>);
   else
-    hipLaunchKernelGGL((router_kernel<1>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream,
-                       static_cast<const uint16_t*>(hidden), static_cast<const uint16_t*>(router_weight), logits,
-                       (int)tokens, (int)n_routed, (int)model_dim);
-  const int st = aklr_moe_fp8_route(logits, correction_bias, tokens, n_routed, topk, num_expert_group, topk_group,
-                                    renormalize, routed_scaling_factor, 1, ids, weights, stream);
-  if (st != AKLR_OK) return st;
+    router(router_kernel<4, 4, 1, 1>);
+  launch_route(nullptr, part, rp.ranges, static_cast<const uint16_t*>(correction_bias), tokens, n_routed,
+               num_expert_group, topk, topk_group, renormalize, routed_scaling_factor, 1, ids, weights, stream);
   return run_experts(static_cast<const uint16_t*>(hidden), tokens, model_dim, inter_dim, E, ids, weights, S,
                      static_cast<const uint8_t*>(w1), w1_scale, static_cast<const uint8_t*>(w2), w2_scale, w_layout,
                      static_cast<uint16_t*>(out), ws, L, stream);
