@@ -114,6 +114,21 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+def host_function(name: str):
+    """The native host path of an op (``aklr_amd._host``): called with a call's args tuple and kwargs dict,
+    it returns the outputs or None for a call the general path has to decide. None when the library itself
+    is not built (the general path says so where it needs it)."""
+    if not Path(LIB_PATH).exists():
+        return None
+    lib()  # checks its ABI version
+    try:
+        from . import _host
+    except ImportError as e:
+        raise NativeLibraryError(f"aklr_amd._host is not built or does not load: run "
+                                 f"`python -c 'import __graft_entry__ as g; g.build()'` ({e})") from e
+    return getattr(_host, name)
+
+
 def digest() -> str:
     lib()
     assert _digest is not None

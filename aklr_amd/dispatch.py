@@ -170,11 +170,14 @@ def on_gpu(*tensors) -> bool:
     return True
 
 
-def api(contract_id: str, run_fn):
+def api(contract_id: str, run_fn, native: str | None = None):
     """Decorator binding an op. The decorated function has the op's exact signature and returns a
     plan object (with ``.variant`` and ``.kernel_ref``) or a FallbackReason; ``run_fn(plan)``
     launches and returns the outputs. The result is the api function, with ``.serving`` and
-    ``.fallback_reason`` of the same signature attached."""
+    ``.fallback_reason`` of the same signature attached. ``native`` names the op's function in
+    ``aklr_amd._host``: a call on GPU tensors goes there first, and comes back here (``.general``) where that
+    function leaves the decision to the plan. A call whose first argument is not on a GPU skips it, so the
+    ops answer without the native library there, as before."""
     import functools
 
     from . import _lib
@@ -200,7 +203,7 @@ def api(contract_id: str, run_fn):
             return served if isinstance(served, FallbackReason) else None
 
         @functools.wraps(plan_fn)
-        def call(*args, **kwargs):
+        def general(*args, **kwargs):
             plan = _plan(*args, **kwargs)
             if isinstance(plan, FallbackReason):
                 trace(contract_id, None, plan)
@@ -209,6 +212,24 @@ def api(contract_id: str, run_fn):
             trace(contract_id, plan.variant, plan.kernel_ref)
             return result
 
+        if native is None:
+            call = general
+        else:
+            host = None
+
+            @functools.wraps(plan_fn)
+            def call(*args, **kwargs):
+                nonlocal host
+                if host is None:
+                    if not (args and getattr(args[0], "is_cuda", False)) or disabled(contract_id):
+                        return general(*args, **kwargs)
+                    host = _lib.host_function(native)
+                    if host is None:
+                        return general(*args, **kwargs)
+                result = host(args, kwargs)
+                return general(*args, **kwargs) if result is None else result
+
+        call.general = general
         call.serving = serving
         call.fallback_reason = fallback_reason
         call.contract_id = contract_id

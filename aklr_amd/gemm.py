@@ -105,7 +105,7 @@ def _run_gemm8(p: _Gemm8Plan):
     return out
 
 
-@api("gemm_a8w8_blockwise_scaled@1.0", _run_gemm8)
+@api("gemm_a8w8_blockwise_scaled@1.0", _run_gemm8, native="gemm_fp8")
 def gemm_a8w8_blockwise_scaled(
     a,
     b,
@@ -229,7 +229,7 @@ def _run_quant_gemm8(p: _QuantGemm8Plan):
     return out
 
 
-@api("quant_gemm_a8w8_blockwise_scaled@1.0", _run_quant_gemm8)
+@api("quant_gemm_a8w8_blockwise_scaled@1.0", _run_quant_gemm8, native="quant_gemm_fp8")
 def quant_gemm_a8w8_blockwise_scaled(x, b, b_scale, bias=None, out_dtype=None, out=None, *,
                                      operand_format="none:none"):
     """``gemm_a8w8_blockwise_scaled(*per_group_quant_fp8(x), b, b_scale, ...)`` in one call, equal bit for
@@ -319,7 +319,7 @@ def _run_gemm4(p: _Gemm4Plan):
     return out
 
 
-@api("gemm_a4w4_mxfp4@1.0", _run_gemm4)
+@api("gemm_a4w4_mxfp4@1.0", _run_gemm4, native="gemm_mxfp4")
 def gemm_a4w4_mxfp4(
     a,
     b,

@@ -60,7 +60,7 @@ def _run_fp8(p: _QuantPlan):
     return q, s
 
 
-@api("per_group_quant_fp8@1.0", _run_fp8)
+@api("per_group_quant_fp8@1.0", _run_fp8, native="quant_fp8")
 def per_group_quant_fp8(x):
     if not _x_ok(x, 128):
         return FallbackReason.OUT_OF_CONTRACT
@@ -79,7 +79,7 @@ def _run_mxfp8(p: _QuantPlan):
     return q, s
 
 
-@api("per_group_quant_mxfp8@1.0", _run_mxfp8)
+@api("per_group_quant_mxfp8@1.0", _run_mxfp8, native="quant_mxfp8")
 def per_group_quant_mxfp8(x):
     if not _x_ok(x, 32):
         return FallbackReason.OUT_OF_CONTRACT
@@ -107,7 +107,7 @@ def _run_mxfp4(p: _QuantPlan):
     return q.view(_FP4X2), s.view(_E8M0)
 
 
-@api("dynamic_mxfp4_quant@1.0", _run_mxfp4)
+@api("dynamic_mxfp4_quant@1.0", _run_mxfp4, native="quant_mxfp4")
 def dynamic_mxfp4_quant(x, shuffle=False):
     if not _x_ok(x, 32, _MAX_HIDDEN_MXFP4) or shuffle not in (True, False):
         return FallbackReason.OUT_OF_CONTRACT
