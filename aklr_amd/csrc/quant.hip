@@ -177,30 +177,45 @@ __device__ __forceinline__ int64_t shuffled_scale_offset(int64_t row, int64_t co
   return ((((r0 * (pc >> 3) + c0) * 4 + c3) * 16 + r2) * 2 + c2) * 2 + r1;
 }
 
-// dynamic_mxfp4_quant (aklr/ops/fused_moe/reference.py:21-37). One 256-thread workgroup per row, the
-// chunks of the MXFP8 kernel. With a shuffled scale layout the grid also covers the padding
-// rows/columns, whose scale bytes are written as 0x00.
+// dynamic_mxfp4_quant (aklr/ops/fused_moe/reference.py:21-37). The chunks of the MXFP8 kernel; a workgroup
+// takes 4 * CH consecutive chunks of one row, wave w its chunks w, w + 4, ... With a shuffled scale layout
+// the rows go up to the next multiple of 32 and the columns to the padded ones, whose scale bytes are 0x00
+// (they share dwords with real ones), and the workgroups past those rows fill the whole 32-row groups of
+// padding, which are contiguous, with 16-byte stores.
+//
+// CH = 8 keeps 8 loads in flight a wave for the large inputs, which HBM bounds. While all chunks fit the
+// chip at one per wave (kMxfp4Waves) a call is latency alone -- launch, one load, one conversion -- and
+// CH = 1 spreads a row over workgroups instead of walking it: 8 x 8192 shuffled 3.05 -> 2.1 us, 300 x 8192 4.05 -> 3.3 (there the
+// byte stores of 248 padding rows, now 14 workgroups of wide ones, took part of it too).
+constexpr int64_t kMxfp4Waves = 8192;
+
+template <int CH>
 __global__ __launch_bounds__(256) void quant_mxfp4_kernel(const uint16_t* __restrict__ x, int64_t xs,
                                                           uint8_t* __restrict__ q, uint8_t* __restrict__ scales,
-                                                          int64_t rows, int64_t cols, int shuffled,
-                                                          int64_t pad_cols) {
+                                                          int64_t rows, int64_t cols, int shuffled, int64_t pad_cols,
+                                                          int64_t on_rows, int64_t fill_from, int64_t fill_end) {
   const int64_t row = blockIdx.x;
+  if (row >= on_rows) {  // padding: 4 KiB of zero scale bytes a workgroup
+    const int64_t at = fill_from + (row - on_rows) * 4096 + threadIdx.x * 16;
+    if (blockIdx.y == 0 && at < fill_end) *reinterpret_cast<u32x4*>(scales + at) = u32x4{0, 0, 0, 0};
+    return;
+  }
   const int64_t groups = cols >> 5;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int part = lane & 3;
   const int64_t gcount = shuffled ? pad_cols : groups;
   const int64_t chunks = (gcount + 15) >> 4;
   const bool row_on = row < rows;
-  for (int64_t c0 = w; c0 < chunks; c0 += 4 * kChunks32) {
-  u32x4 v[kChunks32];
+  const int64_t c0 = (int64_t)blockIdx.y * (4 * CH) + w;
+  u32x4 v[CH];
 #pragma unroll
-  for (int i = 0; i < kChunks32; ++i) {
+  for (int i = 0; i < CH; ++i) {
     const int64_t g = ((c0 + 4 * i) << 4) + (lane >> 2);
     v[i] = u32x4{0, 0, 0, 0};
     if (row_on && c0 + 4 * i < chunks && g < groups) v[i] = ld16_nt(x + row * xs + g * 32 + part * 8);
   }
 #pragma unroll
-  for (int i = 0; i < kChunks32; ++i) {
+  for (int i = 0; i < CH; ++i) {
     if (c0 + 4 * i >= chunks) break;  // wave-uniform
     const int64_t g = ((c0 + 4 * i) << 4) + (lane >> 2);
     const Group32 gv = unpack_group32(v[i]);
@@ -231,7 +246,6 @@ __global__ __launch_bounds__(256) void quant_mxfp4_kernel(const uint16_t* __rest
       else
         scales[row * groups + g] = (uint8_t)sbyte;
     }
-  }
   }
 }
 
@@ -308,9 +322,22 @@ extern "C" int aklr_dynamic_mxfp4_quant(const void* x, int64_t x_row_stride, uin
   const int64_t pad_rows = shuffled ? (n_tokens + 255) / 256 * 256 : n_tokens;
   const int64_t pad_cols = shuffled ? (groups + 7) / 8 * 8 : groups;
   if (pad_rows > 0x7FFFFFFF) return AKLR_ERR_INVALID_ARGUMENT;
-  const dim3 grid((unsigned)pad_rows);
-  hipLaunchKernelGGL(quant_mxfp4_kernel, grid, dim3(256), 0, stream, static_cast<const uint16_t*>(x),
-                     x_row_stride, quantized, scales, n_tokens, hidden_size, shuffled ? 1 : 0, pad_cols);
+  const int64_t chunks = (pad_cols + 15) / 16;
+  const bool spread = (shuffled ? (n_tokens + 31) / 32 * 32 : n_tokens) * chunks <= kMxfp4Waves;
+  // the wide fill needs 16-byte alignment; without it the padding rows take the rows' byte stores
+  const bool wide = (reinterpret_cast<uintptr_t>(scales) & 15u) == 0;
+  const int64_t on_rows = shuffled && wide ? (n_tokens + 31) / 32 * 32 : pad_rows;
+  const int64_t fill_from = on_rows * pad_cols, fill_end = pad_rows * pad_cols;
+  const int64_t blocks = on_rows + (fill_end - fill_from + 4095) / 4096;
+  const dim3 grid((unsigned)blocks, (unsigned)((chunks + (spread ? 4 : 32) - 1) / (spread ? 4 : 32)));
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, static_cast<const uint16_t*>(x), x_row_stride, quantized, scales,
+                       n_tokens, hidden_size, shuffled ? 1 : 0, pad_cols, on_rows, fill_from, fill_end);
+  };
+  if (spread)
+    go(quant_mxfp4_kernel<1>);
+  else
+    go(quant_mxfp4_kernel<kChunks32>);
   AKLR_LAUNCH_CHECK();
   return AKLR_OK;
 }
