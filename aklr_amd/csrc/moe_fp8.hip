@@ -36,6 +36,7 @@ constexpr int kClasses = 3;
 constexpr int kMinTM = 64;
 __host__ __device__ constexpr int class_rows(int k) { return k == 0 ? 256 : (k == 1 ? 128 : 64); }
 constexpr int kTN = 256;   // weight rows per GEMM tile
+constexpr int kItemSteps = 16;  // K steps of a DOWN item of several tiles (its b_scale rows: 2 values a step)
 constexpr int kMaxExperts = 2048;  // expert slots the align kernel's LDS holds
 constexpr float kFp32Tiny = 1.17549435e-38f;
 
@@ -549,8 +550,15 @@ constexpr int kMoeSmemBytes =
         : (MoeSmem<128>::kBytes > MoeSmem<64>::kBytes ? MoeSmem<128>::kBytes : MoeSmem<64>::kBytes);
 static_assert(kMoeSmemBytes <= 160 * 1024, "LDS");
 
+//
+// DOWN items of the 64- and 128-row classes take `tiles` consecutive weight tiles from pn on, in one stream of
+// tiles * KB steps through the ring (the 256-row class, whose accumulators leave no registers for it, one): a tile's results are stored between two steps while the next tile's stages are in flight. On short
+// K an item of one tile is mostly its own start (a ticket, the block's entry, the b_scale rows and the first
+// stages, one after the other): 128 tokens on 256 experts of 7168 x 256 (2 K blocks, 28 tiles) took 100 us
+// for 460 MB of weights, and 75 in items of 6 tiles. From 16 K blocks on items keep one tile (32 steps an
+// item instead of 16: 4096 tokens at 2048, 3420 -> 3470 us a call, the last items end too far apart).
 template <int MODE, bool PRE, int TM>
-__device__ __forceinline__ void moe_item(const MoeGemmArgs& p, uint8_t* smem, int cls, int blk, int pn) {
+__device__ __forceinline__ void moe_item(const MoeGemmArgs& p, uint8_t* smem, int cls, int blk, int pn, int tiles) {
   using L = MoeSmem<TM>;
   constexpr int TN = kTN, S = L::S;
   constexpr int MT = TM / 32, NT = TN / 64;
@@ -558,11 +566,12 @@ __device__ __forceinline__ void moe_item(const MoeGemmArgs& p, uint8_t* smem, in
   constexpr int kLoads = AI + BI + 1;
   constexpr int kScaleWaves = TM / 64;
   constexpr int kStageA = L::kStageA, kStageB = L::kStageB;
+  constexpr bool kMany = MODE == kDown && TM < 256;  // several tiles an item
   uint8_t* sA = smem + L::kA;
   uint8_t* sB = smem + L::kB;
   float* sS = reinterpret_cast<float*>(smem + L::kS);
   float* sDummy = reinterpret_cast<float*>(smem + L::kDummy);
-  float (*sSB)[512] = reinterpret_cast<float (*)[512]>(smem + L::kSB);
+  float* sSB = reinterpret_cast<float*>(smem + L::kSB);
   float (*sAmax)[MT][16][4] = reinterpret_cast<float (*)[MT][16][4]>(smem + L::kAmax);
 
   const int lane = threadIdx.x & 63;
@@ -575,7 +584,9 @@ __device__ __forceinline__ void moe_item(const MoeGemmArgs& p, uint8_t* smem, in
   const int64_t kt32 = p.K >> 5;
   {
     const int bi = cls * p.blk_cap + blk;
-    const int e = p.blk_expert[bi], row0 = p.blk_row[bi], rows = p.blk_rows[bi];
+    // in SGPRs: the loads' descriptors are made from them
+    const int e = __builtin_amdgcn_readfirstlane(p.blk_expert[bi]), row0 = __builtin_amdgcn_readfirstlane(p.blk_row[bi]),
+              rows = __builtin_amdgcn_readfirstlane(p.blk_rows[bi]);
 
     // A: wave w moves tile rows [w*TM/8, (w+1)*TM/8) in slabs of 8; waves below kScaleWaves also move
     // a_scale rows [64w, 64w + 64), the others an empty load (same count per wave).
@@ -618,9 +629,14 @@ __device__ __forceinline__ void moe_item(const MoeGemmArgs& p, uint8_t* smem, in
     const uint32_t lds_a = lds_addr(&sA[w * (TM / 8) * 128]), lds_b = lds_addr(&sB[w * 32 * 128]);
     const uint32_t lds_s = scale_wave ? lds_addr(&sS[w * 64]) : lds_addr(&sDummy[w * 64]);
     const uint32_t lds_s_step = scale_wave ? TM * 4 : 0;
-    auto issue = [&](int kb, int st) {
-      const bool on = kb < KB;
-      const uint32_t ak = (uint32_t)kb * 128u, bk = PRE ? (uint32_t)kb * 2048u : (uint32_t)kb * 128u;
+    // the next stage to load: K block ikb of the item's tile itile (rows past N lie past the descriptor)
+    int ikb = 0, itile = 0;
+    const int n_tiles = kMany ? tiles : 1;
+    auto issue = [&](int st) {
+      const int kb = ikb;
+      const bool on = itile < n_tiles;
+      const uint32_t ak = (uint32_t)kb * 128u;
+      const uint32_t bk = (PRE ? (uint32_t)kb * 2048u : (uint32_t)kb * 128u) + (kMany ? (uint32_t)itile * (uint32_t)(TN * p.K) : 0u);
 #pragma unroll
       for (int j = 0; j < AI; ++j)
         lds_dma16(ars, lds_a + st * kStageA + j * 1024, on && a_off[j] != kOobOffset ? a_off[j] + ak : kOobOffset);
@@ -628,18 +644,22 @@ __device__ __forceinline__ void moe_item(const MoeGemmArgs& p, uint8_t* smem, in
       for (int j = 0; j < BI; ++j)
         lds_dma16(brs, lds_b + st * kStageB + j * 1024, on && b_off[j] != kOobOffset ? b_off[j] + bk : kOobOffset);
       lds_dma4(sars, lds_s + st * lds_s_step, on && sa_off != kOobOffset ? sa_off + (uint32_t)kb * sa_kstep : kOobOffset);
+      if (++ikb == KB) {
+        ikb = 0;
+        ++itile;
+      }
     };
 
     // b_scale rows of the tile over K: GATEUP gate block pn and up block I/128 + pn; DOWN the
-    // tile's two 128-row blocks.
+    // tiles' two 128-row blocks each, tile after tile (they are consecutive rows).
     {
       const float* sbe = p.sb + (int64_t)e * p.sb_stride;
-      const int last = (p.N - 1) >> 7;
-      const int r0 = MODE == kGateUp ? pn : min(2 * pn, last);
-      const int r1 = MODE == kGateUp ? (p.I >> 7) + pn : min(2 * pn + 1, last);
-      for (int i = threadIdx.x; i < 2 * KB; i += 512) {
-        const int r = i >= KB ? 1 : 0, kk = i - r * KB;
-        sSB[r][kk] = sbe[(int64_t)(r ? r1 : r0) * KB + kk];
+      if (MODE == kGateUp) {
+        for (int i = threadIdx.x; i < 2 * KB; i += 512)
+          sSB[i] = sbe[(int64_t)(i >= KB ? (p.I >> 7) + pn : pn) * KB + (i >= KB ? i - KB : i)];
+      } else {
+        const int last = ((p.N - 1) >> 7) * KB + KB - 1 - 2 * pn * KB;  // the expert's last value, from the first row
+        for (int i = threadIdx.x; i < 2 * KB * n_tiles; i += 512) sSB[i] = sbe[(int64_t)2 * pn * KB + min(i, last)];
       }
     }
 
@@ -665,16 +685,16 @@ __device__ __forceinline__ void moe_item(const MoeGemmArgs& p, uint8_t* smem, in
       pend[j] = f32x4{0.f, 0.f, 0.f, 0.f};
       pend_s[j] = 0.f;
     }
-    auto compute = [&](int kb, int st) {
+    auto compute = [&](int kb, int tile, int st) {
       const uint8_t* A = sA + st * kStageA;
       const uint8_t* B = sB + st * kStageB;
       const float* SA = sS + st * TM + wm * (TM / 2) + li;
       float sbv[2];
       if (MODE == kGateUp) {
-        sbv[0] = sSB[0][kb];
-        sbv[1] = sSB[1][kb];
+        sbv[0] = sSB[kb];
+        sbv[1] = sSB[KB + kb];
       } else {
-        sbv[0] = sbv[1] = sSB[wn >> 1][kb];
+        sbv[0] = sbv[1] = sSB[(kMany ? 2 * tile + (wn >> 1) : wn >> 1) * KB + kb];
       }
       auto read_a = [&](int mt) {
         return cat(*reinterpret_cast<const u32x4*>(A + a_row + swz_lo + mt * 2048),
@@ -728,24 +748,60 @@ __device__ __forceinline__ void moe_item(const MoeGemmArgs& p, uint8_t* smem, in
       }
     };
 
+    // the last folds of a tile, then (DOWN) y rows in sorted order, bf16; lane pairs swap halves for 16-byte
+    // stores (see the dense kernel)
+    auto finish_folds = [&]() {
 #pragma unroll
-    for (int s = 0; s < S - 1; ++s) issue(s, s);
+      for (int j = 0; j < kLag; ++j) {
+        const int u = kT - kLag + j;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[tmt(u)][tnt(u)][r] = fmaf(pend[j][r], pend_s[j], acc[tmt(u)][tnt(u)][r]);
+      }
+    };
+    auto store_y = [&](int tile) {
+      const int col_s = (pn + tile) * TN + wn * 64 + (g & 1) * 16 + (g >> 1) * 8;
+#pragma unroll
+      for (int nt = 0; nt < NT; nt += 2)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          const f32x4 xv = acc[mt][nt], yv = acc[mt][nt + 1];
+          const uint32_t x0 = pack_bf16x2(xv[0], xv[1]), x1 = pack_bf16x2(xv[2], xv[3]);
+          const uint32_t y0 = pack_bf16x2(yv[0], yv[1]), y1 = pack_bf16x2(yv[2], yv[3]);
+          const auto s0 = __builtin_amdgcn_permlane16_swap(x0, y0, false, false);
+          const auto s1 = __builtin_amdgcn_permlane16_swap(x1, y1, false, false);
+          const u32x4 v = {s0[0], s1[0], s0[1], s1[1]};
+          const int tr = wm * (TM / 2) + mt * 16 + li, col = col_s + nt * 16;
+          if (tr < rows && col < p.N) *reinterpret_cast<u32x4*>(p.y + (int64_t)(row0 + tr) * p.N + col) = v;
+        }
+    };
+
+#pragma unroll
+    for (int s = 0; s < S - 1; ++s) issue(s);
     int st = 0, st_fill = S - 1;
-    for (int kb = 0; kb < KB; ++kb) {
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * kLoads) : "memory");
-      __syncthreads();
-      issue(kb + S - 1, st_fill);
-      compute(kb, st);
-      st = st + 1 == S ? 0 : st + 1;
-      st_fill = st_fill + 1 == S ? 0 : st_fill + 1;
+    for (int tile = 0; tile < n_tiles; ++tile) {
+      if (kMany && tile > 0) {
+        // the tile before this one; its stores are younger than the stages in flight, so the next waits
+        // cover those stages and some of the stores
+        finish_folds();
+        store_y(tile - 1);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < kLag; ++j) pend[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      for (int kb = 0; kb < KB; ++kb) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * kLoads) : "memory");
+        __syncthreads();
+        issue(st_fill);
+        compute(kb, tile, st);
+        st = st + 1 == S ? 0 : st + 1;
+        st_fill = st_fill + 1 == S ? 0 : st_fill + 1;
+      }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-    for (int j = 0; j < kLag; ++j) {
-      const int u = kT - kLag + j;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[tmt(u)][tnt(u)][r] = fmaf(pend[j][r], pend_s[j], acc[tmt(u)][tnt(u)][r]);
-    }
+    finish_folds();
 
     if (MODE == kGateUp) {
       // h = bf16(silu(gate) * up), kept in the gate tiles' registers; per row, e4m3 at scale
@@ -787,21 +843,7 @@ __device__ __forceinline__ void moe_item(const MoeGemmArgs& p, uint8_t* smem, in
         }
       }
     } else {
-      // y rows in sorted order, bf16; lane pairs swap halves for 16-byte stores (see the dense kernel)
-      const int col_s = pn * TN + wn * 64 + (g & 1) * 16 + (g >> 1) * 8;
-#pragma unroll
-      for (int nt = 0; nt < NT; nt += 2)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          const f32x4 xv = acc[mt][nt], yv = acc[mt][nt + 1];
-          const uint32_t x0 = pack_bf16x2(xv[0], xv[1]), x1 = pack_bf16x2(xv[2], xv[3]);
-          const uint32_t y0 = pack_bf16x2(yv[0], yv[1]), y1 = pack_bf16x2(yv[2], yv[3]);
-          const auto s0 = __builtin_amdgcn_permlane16_swap(x0, y0, false, false);
-          const auto s1 = __builtin_amdgcn_permlane16_swap(x1, y1, false, false);
-          const u32x4 v = {s0[0], s1[0], s0[1], s1[1]};
-          const int tr = wm * (TM / 2) + mt * 16 + li, col = col_s + nt * 16;
-          if (tr < rows && col < p.N) *reinterpret_cast<u32x4*>(p.y + (int64_t)(row0 + tr) * p.N + col) = v;
-        }
+      store_y(n_tiles - 1);
     }
   }
 }
@@ -820,9 +862,17 @@ template <int MODE, bool PRE>
 __global__ __launch_bounds__(512) void moe_gemm_kernel(MoeGemmArgs p) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kMoeSmemBytes];
   __shared__ int ticket;
-  const int tn = p.tiles_n;
   const int n0 = p.nblk[0], n1 = p.nblk[1], n2 = p.nblk[2];
-  const int heavy = n0 * tn, c1 = n1 * tn, items = heavy + c1 + n2 * tn;
+  // weight tiles per item (DOWN): up to kItemSteps K steps, while four items a CU are left
+  int per = 1;
+  if (MODE == kDown) {
+    per = min(kItemSteps / (p.K >> 7), (int)((int64_t)(n0 + n1 + n2) * p.tiles_n / (4 * (int)gridDim.x)));
+    per = per < 1 ? 1 : per;
+    const int groups = (p.tiles_n + per - 1) / per;
+    per = (p.tiles_n + groups - 1) / groups;  // the same number of items, evenly filled
+  }
+  const int tn = (p.tiles_n + per - 1) / per;  // items of a 64- or 128-row block
+  const int heavy = n0 * p.tiles_n, c1 = n1 * tn, items = heavy + c1 + n2 * tn;
   for (;;) {
     __syncthreads();  // every wave is done with the previous item's LDS and has read the ticket
     if (threadIdx.x == 0) ticket = atomicAdd(p.tickets, 1);
@@ -831,13 +881,13 @@ __global__ __launch_bounds__(512) void moe_gemm_kernel(MoeGemmArgs p) {
     if (t >= items) break;
     const int hk = (int)((int64_t)t * heavy / items);  // 256-row items before ticket t
     if ((int64_t)(t + 1) * heavy / items > hk) {
-      moe_item<MODE, PRE, 256>(p, smem, 0, hk / tn, hk % tn);
+      moe_item<MODE, PRE, 256>(p, smem, 0, hk / p.tiles_n, hk % p.tiles_n, 1);
     } else {
-      const int i = t - hk;
+      const int i = t - hk, pn = i % tn * per, tiles = min(per, p.tiles_n - pn);  // c1 is a multiple of tn
       if (i < c1)
-        moe_item<MODE, PRE, 128>(p, smem, 1, i / tn, i % tn);
+        moe_item<MODE, PRE, 128>(p, smem, 1, i / tn, pn, tiles);
       else
-        moe_item<MODE, PRE, 64>(p, smem, 2, (i - c1) / tn, (i - c1) % tn);
+        moe_item<MODE, PRE, 64>(p, smem, 2, (i - c1) / tn, pn, tiles);
     }
   }
 }
