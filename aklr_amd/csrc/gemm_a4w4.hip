@@ -656,11 +656,14 @@ __global__ __launch_bounds__(512) void gemm4_lds_kernel(Gemm4Args p) {
   static_assert(TM % 64 == 0 && TN % 128 == 0 && S >= 2, "tile shape");
   constexpr int MT = TM / 32, NT = TN / 64, AI = TM / 64, BI = TN / 64;
   constexpr int kLoads = AI + BI + 2;  // + one A-scale and one B-scale load
+  constexpr bool kTwo = TM == 256 && PRE;  // two barriers a step (below)
+  constexpr int AH = kTwo ? AI / 2 : AI;
+  constexpr int kFirst = BI + 2 + AH;  // kTwo: the loads of a stage that go out first: B, the scales, A's first half
   constexpr int kStageA = TM * 128, kStageB = TN * 128, kScaleA = TM * 8, kScaleB = TN * 8;
   __shared__ __attribute__((aligned(1024))) uint8_t sA[S * kStageA];
   __shared__ __attribute__((aligned(1024))) uint8_t sB[S * kStageB];
-  __shared__ __attribute__((aligned(16))) uint8_t sSA[S * kScaleA];
-  __shared__ __attribute__((aligned(16))) uint8_t sSB[S * kScaleB];
+  __shared__ __attribute__((aligned(16))) uint8_t sSA[(S + kTwo) * kScaleA];
+  __shared__ __attribute__((aligned(16))) uint8_t sSB[(S + kTwo) * kScaleB];
   __shared__ __attribute__((aligned(16))) uint32_t sDummy[8 * 64];
   __shared__ unsigned arrive_slot;
 
@@ -695,10 +698,15 @@ __global__ __launch_bounds__(512) void gemm4_lds_kernel(Gemm4Args p) {
   const i32x4 brs = make_rsrc_words(p.b + b_base, clamp_bytes(b_total - b_base));
   const int lr = lane >> 3, lp = lane & 7;
   const int c = lp ^ lr;
+  // A in slabs of 8 rows, AI per wave. kTwo: in two halves, half h the h-th half of the rows of each of the
+  // tile's two wave rows, dealt to the waves in turn.
   uint32_t a_off[AI], b_off[BI];
+  int a_slab[AI];
 #pragma unroll
   for (int j = 0; j < AI; ++j) {
-    const int r = w * (TM / 8) + j * 8 + lr;
+    const int i = (j % AH) * 8 + w;
+    a_slab[j] = kTwo ? (i / (TM / 32)) * (TM / 16) + (j / AH) * (TM / 32) + i % (TM / 32) : w * AI + j;
+    const int r = a_slab[j] * 8 + lr;
     a_off[j] = m0 + r < p.m ? (uint32_t)(r * p.lda + c * 16) : kOobOffset;
   }
 #pragma unroll
@@ -729,7 +737,7 @@ __global__ __launch_bounds__(512) void gemm4_lds_kernel(Gemm4Args p) {
     sb_off = sb_wave && rb < p.n ? (uint32_t)((int64_t)rb * p.lds_b + (lane & 1) * 4) : kOobOffset;
     sa_step = sb_step = 8;
   }
-  const uint32_t lds_a = lds_addr(&sA[w * (TM / 8) * 128]), lds_b = lds_addr(&sB[w * (TN / 8) * 128]);
+  const uint32_t lds_a = lds_addr(&sA[kTwo ? 0 : w * (TM / 8) * 128]), lds_b = lds_addr(&sB[w * (TN / 8) * 128]);
   const uint32_t lds_sa = sa_wave ? lds_addr(&sSA[w * 256]) : lds_addr(&sDummy[w * 64]);
   const uint32_t lds_sb = sb_wave ? lds_addr(&sSB[w * 256]) : lds_addr(&sDummy[w * 64]);
   const uint32_t lds_sa_step = sa_wave ? kScaleA : 0, lds_sb_step = sb_wave ? kScaleB : 0;
@@ -793,16 +801,147 @@ __global__ __launch_bounds__(512) void gemm4_lds_kernel(Gemm4Args p) {
     }
   };
 
+  if constexpr (kTwo) {
+    // Two barriers a step, so that loads go out 1.5 steps before they are needed although LDS holds two
+    // stages. The step's B fragments are in registers when it begins, its A fragments stream one row of
+    // tiles ahead, and stage ks + S follows stage ks into its slot in two parts: B, the scales (in a slot
+    // more of their own, since the step's last scale reads come later) and A's first half at the barrier
+    // before row MT/2 - 1, when the rows up to there are in registers; A's second half at the barrier before
+    // the last row. That one also publishes the next step's B and first A half, so the last row's MFMAs
+    // cover the reads of the next step's first fragments. With one barrier at the head of each step the
+    // loads had one step to land in, and every wave waited out the LDS latency of its first fragments there:
+    // at 4096 x 8192 x 8192 loads and fragment reads without MFMAs took 131 us of the 145, and take 109 of
+    // 139 so. What is left is mostly the matrix cores at the clock the chip holds under them: MFMAs alone
+    // take 96. Before -> now, us: 512 x 10240 x 8192 43.3 -> 38.5, 4096 x 10240 x 8192 194.3 -> 189.9,
+    // 4096 x 57344 x 8192 980 -> 944. Tiles of 128 rows lose (64 x 8192 x 28672 34.2 -> 34.9, 200 x 4096 x
+    // 4096 13.6 -> 14.6: half the MFMAs behind each barrier), and so do row-major weights (512 x 10240 x 8192
+    // 53.3 -> 55.1), so those keep the one barrier.
+    // Load i of stage ks: B, the scales, A's first half, then A's second half. The K offset rides soffset,
+    // and a stage past the range goes through a descriptor of no bytes (zeros, no memory traffic).
+    auto issue_one = [&](int i, int ks, int st, int sc) {
+      const bool on = ks < ks_end;
+      if (i < BI) {
+        i32x4 r = brs;
+        r[2] = on ? r[2] : 0;
+        lds_dma16_so(r, lds_b + st * kStageB + i * 1024, b_off[i < BI ? i : 0], PRE ? (uint32_t)ks * 2048u : (uint32_t)ks * 128u);
+      } else if (i == BI) {
+        i32x4 r = sars;
+        r[2] = on ? r[2] : 0;
+        lds_dma4_so(r, lds_sa + sc * lds_sa_step, sa_off, (uint32_t)ks * sa_step);
+      } else if (i == BI + 1) {
+        i32x4 r = sbrs;
+        r[2] = on ? r[2] : 0;
+        lds_dma4_so(r, lds_sb + sc * lds_sb_step, sb_off, (uint32_t)ks * sb_step);
+      } else {
+        const int j = i - BI - 2 >= 0 && i - BI - 2 < AI ? i - BI - 2 : 0;
+        i32x4 r = ars;
+        r[2] = on ? r[2] : 0;
+        lds_dma16_so(r, lds_a + st * kStageA + a_slab[j] * 1024, a_off[j], (uint32_t)ks * 128u);
+      }
+    };
+
+    const int swz0 = (g ^ (li & 7)) << 4, swz1 = ((4 + g) ^ (li & 7)) << 4;
+    struct Frag {  // one 16-row tile of one K step: the codes of both MFMAs and their scale words
+      u32x4 q[2];
+      uint32_t s[2];
+    };
+    auto read_a = [&](int st, int sl, int mt) {
+      const uint8_t* const q = sA + st * kStageA + a_row + mt * 2048;
+      const uint8_t* const sc = sSA + sl * kScaleA + sa_word;
+      Frag f;
+      f.q[0] = *reinterpret_cast<const u32x4*>(q + swz0);
+      f.q[1] = *reinterpret_cast<const u32x4*>(q + swz1);
+      if (SSHUF) {
+        f.s[0] = f.s[1] = *reinterpret_cast<const uint32_t*>(sc + (mt >> 1) * 256);
+      } else {
+        const u32x2 w2 = *reinterpret_cast<const u32x2*>(sc + mt * 128);
+        f.s[0] = w2[0];
+        f.s[1] = w2[1];
+      }
+      return f;
+    };
+    auto read_b = [&](int st, int sl, int nt) {
+      const uint8_t* const q = sB + st * kStageB + b_row + nt * 2048;
+      const uint8_t* const sc = sSB + sl * kScaleB + sb_word;
+      Frag f;
+      f.q[0] = *reinterpret_cast<const u32x4*>(q + swz0);
+      f.q[1] = *reinterpret_cast<const u32x4*>(q + swz1);
+      if (SSHUF) {
+        f.s[0] = f.s[1] = *reinterpret_cast<const uint32_t*>(sc + (nt >> 1) * 256);
+      } else {
+        const u32x2 w2 = *reinterpret_cast<const u32x2*>(sc + nt * 128);
+        f.s[0] = w2[0];
+        f.s[1] = w2[1];
+      }
+      return f;
+    };
+    // the scale byte of MFMA j for tile i: shuffled words hold both MFMAs of a tile pair, row-major ones the
+    // four lane groups of one MFMA
+    auto scale_of = [&](const Frag& f, int j, int i) { return (int)(f.s[j] >> (SSHUF ? 8 * (2 * j + (i & 1)) : 8 * g)); };
+
+    Frag bf[NT], cur, nxt;
+    auto mfma = [&](int mt, int nt, int j) {
+      acc[mt][nt] = mfma16x128_scaled<kFp4, 0, 0>(fp4_frag(bf[nt].q[j]), fp4_frag(cur.q[j]), acc[mt][nt],
+                                                  scale_of(bf[nt], j, nt), scale_of(cur, j, mt));  // lane: row li, cols 4g..
+    };
+    int st = 0, sl = 0;  // the step's slot, and its scales' slot
 #pragma unroll
-  for (int s = 0; s < S - 1; ++s) issue(ks_begin + s, s);
-  int st = 0, st_fill = S - 1;
-  for (int ks = ks_begin; ks < ks_end; ++ks) {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * kLoads) : "memory");
-    __syncthreads();
-    issue(ks + S - 1, st_fill);
-    compute(st);
-    st = st + 1 == S ? 0 : st + 1;
-    st_fill = st_fill + 1 == S ? 0 : st_fill + 1;
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) issue_one(i, ks_begin + s, s, s);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(S * kLoads - kFirst) : "memory");
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) bf[nt] = read_b(0, 0, nt);
+    nxt = read_a(0, 0, 0);
+    for (int ks = ks_begin; ks < ks_end; ++ks) {
+      const int st_next = st + 1 == S ? 0 : st + 1, sl_next = sl == S ? 0 : sl + 1, sl_fill = sl == 0 ? S : sl - 1;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const bool mid = mt == MT / 2 - 1, last = mt + 1 == MT;
+        cur = nxt;
+        if (mid || last)
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 1) * kLoads) : "memory");
+        nxt = last ? read_a(st_next, sl_next, 0) : read_a(st, sl, mt + 1);
+        __builtin_amdgcn_sched_barrier(0);  // left alone, the scheduler reads each fragment just before its MFMAs
+#pragma unroll
+        for (int q = 0; q < NT; q += 2) {
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              mfma(mt, q + u, j);
+              // this MFMA's share of the barrier's loads
+              const int slot = 2 * q + 2 * j + u, from = mid ? 0 : kFirst, count = mid ? kFirst : AH;
+              if (mid || last) {
+#pragma unroll
+                for (int i = 0; i < kLoads; ++i)
+                  if (i >= from && i < from + count && (i - from) * (2 * NT) / count == slot)
+                    issue_one(i, ks + S, st, sl_fill);
+              }
+            }
+          if (last) {
+            bf[q] = read_b(st_next, sl_next, q);
+            bf[q + 1] = read_b(st_next, sl_next, q + 1);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      st = st_next;
+      sl = sl_next;
+    }
+  } else {
+#pragma unroll
+    for (int s = 0; s < S - 1; ++s) issue(ks_begin + s, s);
+    int st = 0, st_fill = S - 1;
+    for (int ks = ks_begin; ks < ks_end; ++ks) {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * kLoads) : "memory");
+      __syncthreads();
+      issue(ks + S - 1, st_fill);
+      compute(st);
+      st = st + 1 == S ? 0 : st + 1;
+      st_fill = st_fill + 1 == S ? 0 : st_fill + 1;
+    }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
