@@ -6,11 +6,12 @@
 // scale of that row and 32-block, and the atom applies the scales itself. No VALU fold: the MFMA
 // accumulates straight into the fp32 result.
 //
-// * skinny (m <= 16, and 16 < m <= 32 with unaligned row-major scales): weight streaming -- a
+// * skinny (m <= 16 but for the stream plans of preshuffled weights, plan_decode4, and 16 < m <= 32 with
+//   unaligned row-major scales): weight streaming -- a
 //   workgroup owns 32 columns and a K range, each wave a contiguous K sub-range with a register ring;
 //   fixed-order wave reduction in LDS, then (when K is also split across workgroups) fp32 partials
 //   summed in split order by the last workgroup to arrive.
-// * stream (16 < m <= 32): the FP8 stream kernel's design -- compute waves stream their own weight
+// * stream (16 < m <= 32, and m <= 16 by plan_decode4): the FP8 stream kernel's design -- compute waves stream their own weight
 //   columns into register rings while a loader wave stages A and its scales in LDS for all of them.
 // * lds (m > 32, k % 256 == 0): the FP8 LDS kernel's tiles and direct-to-LDS ring, K steps of 256
 //   values with the scale bytes staged beside the codes (see gemm4_lds_kernel).
@@ -1007,6 +1008,49 @@ static Skinny4Plan plan_skinny4(int64_t m, int64_t n, int64_t k) {
   return p;
 }
 
+// Decode plan of preshuffled weights (m <= 16), where the skinny plan above does not do: its waves each read
+// A and its scales again, and with 2 K steps in flight a CU holds about 20 KB of weights under way.
+// * K <= 8192, 224 to 1792 column tiles (n = 3584 to 28672): the stream kernel at one row tile, one column
+//   tile a wave, an 8-deep weight ring behind 8 A stages, no K split; one compute wave a workgroup up to 640
+//   tiles (n = 10240), two past that, so that the workgroups stay small and many. us, skinny -> this, m = 1 /
+//   8 / 16: 10240 x 8192 11.8 / 12.2 / 13.6 -> 11.4 / 11.6 / 12.3, 8192 x 8192 10.3 / 11.1 / 11.3 -> 9.9 /
+//   10.2 / 10.4, 4096 x 4096 6.05 / 6.48 / 6.6 -> 5.35 / 5.51 / 5.46, 7168 x 2048 4.59 / 4.84 / 5.16 -> 4.52 /
+//   4.55 / 4.70, 3584 x 448 3.25 / 3.38 / 3.41 -> 2.73 / 2.75 / 2.80, 16384 x 4096 9.6 / 9.9 / 10.5 -> 9.6 /
+//   9.8 / 9.9, 28672 x 8192 25.4 / 26.0 / 28.3 -> 25.4 / 25.3 / 26.6.
+// * wider n, m > 8, K = 4096 to 8192: 224-column workgroups (7 waves of two tiles, a 4-deep ring): 57344 x
+//   8192 at m = 16 47.1 -> 43.5 (at 8 43.2 -> 43.6). Shorter K loses (32768 x 2048 at 16 10.8 -> 11.4).
+// * K > 16384, 112 or more groups of 32 columns: the skinny kernel with 8 waves on the workgroup's K range,
+//   two K splits up to 128 groups: 4096 x 28672 at m = 1 / 8 / 16 18.8 / 19.6 / 20.3 -> 14.9 / 14.9 / 16.0,
+//   8192 x 28672 at 8 / 16 26.5 / 31.9 -> 24.2 / 26.1, 16384 x 28672 48.3 / 67.3 -> 43.9 / 49.5. Past 128
+//   groups one row is even (8192 x 28672 23.3 -> 23.5), and keeps its plan, as does K = 16384 (4608 x 16384
+//   at m = 1 11.9 -> 12.2).
+enum class Decode4 { kSkinny, kStream1, kStream2, kStream14, kSkinny8 };
+static Decode4 plan_decode4(int64_t m, int64_t n, int64_t k) {
+  const int64_t tiles = (n + 15) / 16;
+  if (k <= 8192) {
+    if (tiles >= 224 && tiles <= 1792) return tiles <= 640 ? Decode4::kStream1 : Decode4::kStream2;
+    if (tiles > 1792 && m > 8 && k >= 4096) return Decode4::kStream14;
+  } else if (k > 16384 && n >= 112 * 32 && (m > 1 || n <= 128 * 32)) {
+    return Decode4::kSkinny8;
+  }
+  return Decode4::kSkinny;
+}
+static Skinny4Plan plan_skinny8(int64_t n, int64_t k) {
+  Skinny4Plan p;
+  p.mt = 1;
+  p.nt = 2;
+  p.nw = 8;
+  p.d = 2;
+  p.groups = (int)((n + 31) / 32);
+  const int64_t KS = (k + 127) / 128, s = p.groups <= 128 ? 2 : 1;
+  p.ks_per_split = (int)((KS + s - 1) / s);
+  p.splits = (int)((KS + p.ks_per_split - 1) / p.ks_per_split);
+  return p;
+}
+static size_t skinny4_partial_bytes(const Skinny4Plan& p, int64_t m, int64_t n) {
+  return p.splits > 1 ? (size_t)p.splits * (size_t)round4(m) * (size_t)n * sizeof(float) : 0;
+}
+
 template <int MT, int NT, int D, bool PRE, bool SSHUF>
 static void launch_skinny4(const Gemm4Args& g, const Skinny4Plan& p, hipStream_t s) {
   hipLaunchKernelGGL((gemm4_skinny_kernel<MT, NT, 4, D, PRE, SSHUF>), dim3((unsigned)p.groups, (unsigned)p.splits),
@@ -1139,11 +1183,22 @@ static size_t lds4_partial_bytes(const Lds4Plan& p) {
   return (size_t)p.splits * (size_t)p.tiles * p.tm * p.tn * sizeof(float);
 }
 
+extern "C" int aklr_gemm_a4w4_mxfp4_kernel(int64_t m, int64_t n, int64_t k, int b_layout, int scale_layout) {
+  if (m > kDecode4MaxM) return 2;
+  if (m > 16) return 1;
+  if (b_layout != AKLR_B_PRESHUFFLE_16x16 || scale_layout != AKLR_SCALES_SHUFFLED) return 0;
+  const Decode4 d = plan_decode4(m, n, k);
+  return d == Decode4::kSkinny || d == Decode4::kSkinny8 ? 0 : 1;
+}
+
 extern "C" size_t aklr_gemm_a4w4_mxfp4_workspace_bytes(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k < 64) return 0;
   if (m <= kDecode4MaxM) {  // the stream kernel may be declined at call time: cover the skinny kernel too
-    const Skinny4Plan d = plan_skinny4(m, n, k);
-    size_t need = d.splits > 1 ? (size_t)d.splits * (size_t)round4(m) * (size_t)n * sizeof(float) : 0;
+    size_t need = skinny4_partial_bytes(plan_skinny4(m, n, k), m, n);
+    if (m <= 16 && plan_decode4(m, n, k) == Decode4::kSkinny8) {
+      const size_t pre = skinny4_partial_bytes(plan_skinny8(n, k), m, n);
+      if (pre > need) need = pre;
+    }
     if (m >= kStream4MinM) {
       const Stream4Plan sp = plan_stream4(n, k);
       if (sp.splits > 1 && stream4_partial_bytes(sp) > need) need = stream4_partial_bytes(sp);
@@ -1216,18 +1271,35 @@ extern "C" int aklr_gemm_a4w4_mxfp4(const uint8_t* a, int64_t lda, const uint8_t
     AKLR_LAUNCH_CHECK();
     return AKLR_OK;
   }
+  const Decode4 decode = m <= 16 && g.b_pre && g.scale_shuffled ? plan_decode4(m, n, k) : Decode4::kSkinny;
+  if (decode == Decode4::kStream1 || decode == Decode4::kStream2 || decode == Decode4::kStream14) {
+    const int cols = decode == Decode4::kStream1 ? 16 : (decode == Decode4::kStream2 ? 32 : 224);
+    const dim3 grid((unsigned)((n + cols - 1) / cols));
+    g.ks_per_split = (int)((k + 255) / 256);
+    if (decode == Decode4::kStream1)
+      hipLaunchKernelGGL((gemm4_stream_kernel<1, 1, 1, 8, 8, true, true>), grid, dim3(2 * 64), 0, stream, g);
+    else if (decode == Decode4::kStream2)
+      hipLaunchKernelGGL((gemm4_stream_kernel<1, 1, 2, 8, 8, true, true>), grid, dim3(3 * 64), 0, stream, g);
+    else
+      hipLaunchKernelGGL((gemm4_stream_kernel<1, 2, 7, 4, 8, true, true>), grid, dim3(8 * 64), 0, stream, g);
+    AKLR_LAUNCH_CHECK();
+    return AKLR_OK;
+  }
   if (m <= kDecode4MaxM) {
-    const Skinny4Plan d = plan_skinny4(m, n, k);
+    const Skinny4Plan d = decode == Decode4::kSkinny8 ? plan_skinny8(n, k) : plan_skinny4(m, n, k);
     g.splits = d.splits;
     g.ks_per_split = d.ks_per_split;
     if (d.splits > 1) {
-      const size_t need = kSplitkCounterBytes + (size_t)d.splits * (size_t)round4(m) * (size_t)n * sizeof(float);
+      const size_t need = kSplitkCounterBytes + skinny4_partial_bytes(d, m, n);
       if (!workspace || workspace_bytes < need || !aklr_aligned16(workspace)) return AKLR_ERR_WORKSPACE;
       g.counters = static_cast<uint64_t*>(workspace);
       g.partial = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kSplitkCounterBytes);
     }
     const bool sshuf = scale_layout == AKLR_SCALES_SHUFFLED;
-    if (g.b_pre) sshuf ? launch_skinny4<true, true>(g, d, stream) : launch_skinny4<true, false>(g, d, stream);
+    if (decode == Decode4::kSkinny8)
+      hipLaunchKernelGGL((gemm4_skinny_kernel<1, 2, 8, 2, true, true>), dim3((unsigned)d.groups, (unsigned)d.splits),
+                         dim3(8 * 64), 0, stream, g);
+    else if (g.b_pre) sshuf ? launch_skinny4<true, true>(g, d, stream) : launch_skinny4<true, false>(g, d, stream);
     else sshuf ? launch_skinny4<false, true>(g, d, stream) : launch_skinny4<false, false>(g, d, stream);
     AKLR_LAUNCH_CHECK();
     return AKLR_OK;

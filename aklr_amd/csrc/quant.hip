@@ -185,8 +185,9 @@ __device__ __forceinline__ int64_t shuffled_scale_offset(int64_t row, int64_t co
 //
 // CH = 8 keeps 8 loads in flight a wave for the large inputs, which HBM bounds. While all chunks fit the
 // chip at one per wave (kMxfp4Waves) a call is latency alone -- launch, one load, one conversion -- and
-// CH = 1 spreads a row over workgroups instead of walking it: 8 x 8192 shuffled 3.05 -> 2.1 us, 300 x 8192 4.05 -> 3.3 (there the
-// byte stores of 248 padding rows, now 14 workgroups of wide ones, took part of it too).
+// CH = 1 spreads a row over workgroups instead of walking it: 8 x 8192 shuffled 3.05 -> 2.1 us, 300 x 8192
+// 4.05 -> 3.3 (there the byte stores of 248 padding rows, now 14 workgroups of wide ones, took part of it
+// too); 4096 x 8192 19 us either way.
 constexpr int64_t kMxfp4Waves = 8192;
 
 template <int CH>

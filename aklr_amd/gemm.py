@@ -383,8 +383,10 @@ def gemm_a4w4_mxfp4(
     if not _out_ok(out, m, n, dt, a.device, (a, b, a_scale, b_scale, bias)):
         return _OOC
     pre = variant == "b_shuffled"
-    path = "skinny" if m <= 16 else ("stream" if m <= 32 else "lds")  # as the library picks (aligned scales)
+    b_layout, scale_layout = ((_lib.B_PRESHUFFLE_16x16, _lib.SCALES_SHUFFLED) if pre
+                              else (_lib.B_ROW_MAJOR, _lib.SCALES_ROW_MAJOR))
+    # as the library picks (aligned scales)
+    path = ("skinny", "stream", "lds")[_lib.lib().aklr_gemm_a4w4_mxfp4_kernel(m, n, k, b_layout, scale_layout)]
     return _Gemm4Plan(a, b, a_scale, b_scale, bias, out, dt, m, n, k,
-                      _lib.B_PRESHUFFLE_16x16 if pre else _lib.B_ROW_MAJOR,
-                      _lib.SCALES_SHUFFLED if pre else _lib.SCALES_ROW_MAJOR, variant,
+                      b_layout, scale_layout, variant,
                       f"aklr_gemm_a4w4_mxfp4:{path}")

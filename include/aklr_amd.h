@@ -193,6 +193,9 @@ int aklr_quant_gemm_a8w8_blockscale(const void* x, int64_t ldx, const void* b, i
  * k % 64 == 0 (k % 128 == 0 is not required), n % 16 == 0.
  */
 size_t aklr_gemm_a4w4_mxfp4_workspace_bytes(int64_t m, int64_t n, int64_t k);
+/* Which kernel a call of these sizes runs: 0 skinny, 1 stream, 2 tiled (LDS; scales as the library's layouts
+ * align them). */
+int aklr_gemm_a4w4_mxfp4_kernel(int64_t m, int64_t n, int64_t k, int b_layout, int scale_layout);
 int aklr_gemm_a4w4_mxfp4(const uint8_t* a, int64_t lda, const uint8_t* b, int64_t ldb, const uint8_t* a_scale,
                          int64_t lds_a, const uint8_t* b_scale, int64_t lds_b, const float* bias, void* out,
                          int64_t ldo, int64_t m, int64_t n, int64_t k, int b_layout, int scale_layout,
