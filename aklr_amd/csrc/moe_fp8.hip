@@ -788,8 +788,12 @@ __device__ __forceinline__ void moe_item(const MoeGemmArgs& p, uint8_t* smem, in
         for (int i = 0; i < MT; ++i)
 #pragma unroll
           for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // both: the next tile folds 0 * pend_s first, and a scale of this tile may be infinite or NaN
 #pragma unroll
-        for (int j = 0; j < kLag; ++j) pend[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < kLag; ++j) {
+          pend[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+          pend_s[j] = 0.f;
+        }
       }
       for (int kb = 0; kb < KB; ++kb) {
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * kLoads) : "memory");
