@@ -167,6 +167,23 @@ static RouterPlan plan_router(int64_t T, int64_t E, int64_t D) {
   return p;
 }
 
+// fp32 partials the scratch of a T-token call holds: at least ranges * T * E of every plan for up to T tokens,
+// so that the size never falls as T grows (ranges does) and a buffer made for the largest batch serves the
+// smaller ones. A plan has one range, T * E partials, or at most 16 with at most 512 workgroups, each a tile.
+static int64_t router_partials(int64_t T, int64_t E) {
+  const auto cut = [E](int64_t t, int64_t tm, int64_t tn) {
+    const int64_t most = 16 * ((t + tm - 1) / tm * tm) * E;
+    return most < 512 * tm * tn ? most : 512 * tm * tn;
+  };
+  int64_t n = T * E;
+  const auto cover = [&n](int64_t v) { n = v > n ? v : n; };
+  const bool wide = T >= 1024 && E > 64;
+  cover(cut(T < 16 ? T : 16, 16, 16));
+  if (T > 16) cover(cut(wide ? 1023 : T, 32, 32));
+  if (wide) cover(cut(T, 64, 256));
+  return n;
+}
+
 // ---------------------------------------------------------------------------------------------
 // route: one wave per token. (value, index) pairs compare by value, then the lower index first; a NaN is
 // never picked. As one 64-bit key: the value's bits in an unsigned order, then the inverted index; 0 marks
@@ -962,7 +979,7 @@ static Workspace layout(int64_t T, int64_t S, int64_t D, int64_t I, int64_t E, i
     o = align256(o + bytes);
     return at;
   };
-  w.part = take(Er ? (size_t)(plan_router(T, Er, D).ranges * T * Er * 4) : 0);
+  w.part = take((size_t)(Er ? router_partials(T, Er) * 4 : 0));
   w.ids = take((size_t)(Er ? R * 4 : 0));
   w.weights = take((size_t)(Er ? R * 4 : 0));
   w.row_of = take((size_t)R * 4);

@@ -101,9 +101,8 @@ def _run_moe(p: _MoePlan):
     out = torch.empty((p.tokens, p.d), dtype=torch.bfloat16, device=dev)
     L = _lib.lib()
     chunks = token_chunks(p.tokens, p.d, p.inter, p.topk + 1)
-    # every chunk size's own need: a smaller call cuts the router's K further, into more partials a token
-    ws_bytes = max(L.aklr_moe_fp8_workspace_bytes(c, p.d, p.inter, p.n_routed + 1, p.topk + 1, p.n_routed)
-                   for c in {e - s for s, e in chunks})
+    most = max(e - s for s, e in chunks)
+    ws_bytes = L.aklr_moe_fp8_workspace_bytes(most, p.d, p.inter, p.n_routed + 1, p.topk + 1, p.n_routed)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     row = p.d * 2  # bytes per hidden / out row
     for s, e in chunks:

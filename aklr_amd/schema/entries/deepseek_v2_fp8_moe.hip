@@ -57,10 +57,8 @@ void run(const at::Tensor& hidden_states, const at::Tensor& router_weight, const
   const int64_t slots = topk + 1;
   const int64_t most = tokens_per_call(d, inter, slots);
   TORCH_CHECK(most >= 1, "deepseek_v2_fp8_moe: dimensions past the kernels' 32-bit offsets");
-  // the first and the last chunk's needs: a smaller call cuts the router's K further, into more partials a token
-  const int64_t first = std::min(t, most), rest = t - (t - 1) / most * most;
-  const size_t ws_bytes = std::max(aklr_moe_fp8_workspace_bytes(first, d, inter, n_routed + 1, slots, n_routed),
-                                   aklr_moe_fp8_workspace_bytes(rest, d, inter, n_routed + 1, slots, n_routed));
+  const int64_t first = std::min(t, most);
+  const size_t ws_bytes = aklr_moe_fp8_workspace_bytes(first, d, inter, n_routed + 1, slots, n_routed);
   at::Tensor ws = aklr_entry::scratch(x, ws_bytes);
   const int64_t row_bytes = d * 2;
   for (int64_t s = 0; s < t; s += most) {

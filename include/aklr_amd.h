@@ -220,7 +220,8 @@ int aklr_gemm_a4w4_mxfp4(const uint8_t* a, int64_t lda, const uint8_t* b, int64_
  * model_dim, inter_dim multiples of 128 (<= 16384); tokens <= 65536; n_routed <= 1024, divisible by
  *   num_expert_group (<= 64) with >= 2 experts per group; topk <= 63.
  * Workspace: aklr_moe_fp8_workspace_bytes(tokens, model_dim, inter_dim, n_routed + 1, topk + 1,
- *   n_routed); no zeroing needed.
+ *   n_routed); no zeroing needed. The size never falls as tokens grows: a buffer for the largest call
+ *   serves the smaller ones.
  */
 size_t aklr_moe_fp8_workspace_bytes(int64_t tokens, int64_t model_dim, int64_t inter_dim, int64_t n_experts,
                                     int64_t slots, int64_t n_router_rows);

@@ -7,6 +7,8 @@ import re
 import subprocess
 from pathlib import Path
 
+import pytest
+
 from aklr_amd import _build, _lib
 
 HEADER = Path(__file__).resolve().parents[1] / "include" / "aklr_amd.h"
@@ -78,6 +80,33 @@ def test_workspace_sizes_are_host_computable(native_lib):
         # of workgroups at most 256 x 256
         assert ws % 1024 == 0 and ws <= 131072 + 8 * up(m, 256) * up(n, 256) * 4
     assert L.aklr_gemm_a4w4_mxfp4_workspace_bytes(1, 10240, 8192) % 4 == 0
+
+
+def _router_partials(t, e, d):
+    """The router's fp32 partials of a call: ranges * t * e, by the plan of moe_fp8.hip (plan_router)."""
+    tm, tn, waves = (16, 16, 4) if t <= 16 else ((32, 32, 4) if t < 1024 or e <= 64 else (64, 256, 1))
+    r = min(16, max(1, 512 // (-(-t // tm) * -(-e // tn))))
+    steps = -(-(d // 32) // (r * waves))
+    return -(-(d // 32) // (steps * waves)) * t * e
+
+
+@pytest.mark.parametrize("d,inter,routed,slots", [(7168, 2048, 256, 9), (1024, 256, 1024, 9), (128, 128, 2, 2),
+                                                  (128, 128, 64, 2), (384, 128, 65, 3), (16384, 128, 257, 9)])
+def test_moe_workspace_never_falls_with_tokens_and_holds_the_partials(native_lib, d, inter, routed, slots):
+    size = native_lib.aklr_moe_fp8_workspace_bytes
+    up = lambda v: -(-v // 256) * 256
+    last = 0
+    tokens = [t for t in list(range(1, 1200)) + list(range(1200, 9000, 7)) + [1 << i for i in range(11, 17)]
+              + [(1 << i) + 1 for i in range(11, 16)]]
+    for t in sorted(set(tokens)):
+        got = size(t, d, inter, routed + 1, slots, routed)
+        if not got:  # past what one call takes
+            break
+        assert got >= last, f"{t} tokens need less than fewer tokens do"
+        last = got
+        # beside the router's partials a call has its ids and weights and what the experts alone need
+        partials = got - size(t, d, inter, routed + 1, slots, 0) - 2 * up(t * slots * 4)
+        assert partials >= 4 * _router_partials(t, routed, d)
 
 
 def test_gemm8_kernel_query(native_lib):
