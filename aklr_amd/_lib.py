@@ -47,6 +47,9 @@ SIGNATURES: dict[str, tuple] = {
     ),
     "aklr_gemm_a4w4_mxfp4_workspace_bytes": (_c_size, [_c_i64, _c_i64, _c_i64]),
     "aklr_gemm_a4w4_mxfp4_kernel": (_c_int, [_c_i64, _c_i64, _c_i64, _c_int, _c_int]),
+    "aklr_gemm_a4w4_mxfp4_tile": (
+        _c_int, [_c_i64, _c_i64, _c_i64, _c_int, ctypes.POINTER(_c_int), ctypes.POINTER(_c_int), ctypes.POINTER(_c_int)],
+    ),
     "aklr_gemm_a4w4_mxfp4": (
         _c_int,
         [_vp, _c_i64, _vp, _c_i64, _vp, _c_i64, _vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int,

@@ -652,19 +652,21 @@ __global__ __launch_bounds__(256) void gemm4_tile_kernel(Gemm4Args p) {
 // contiguous 256-byte chunk, loaded as it is; lane (li, g) then finds its scales for both MFMAs of
 // the step and both 16-row halves in the dword at (16g + li) * 4, byte 2 * mfma + half. Row-major
 // scales are staged as 8 bytes per row (lane pairs load a row's two dwords).
-template <int TM, int TN, int S, bool PRE, bool SSHUF>
+//
+// TWO (256-row tiles of preshuffled weights from kTwoMinK on): two barriers a step, see the loop below.
+constexpr int kTwoMinK = 4096;
+template <int TM, int TN, int S, bool PRE, bool SSHUF, bool TWO>
 __global__ __launch_bounds__(512) void gemm4_lds_kernel(Gemm4Args p) {
-  static_assert(TM % 64 == 0 && TN % 128 == 0 && S >= 2, "tile shape");
+  static_assert(TM % 64 == 0 && TN % 128 == 0 && S >= 2 && (!TWO || (TM == 256 && PRE)), "tile shape");
   constexpr int MT = TM / 32, NT = TN / 64, AI = TM / 64, BI = TN / 64;
   constexpr int kLoads = AI + BI + 2;  // + one A-scale and one B-scale load
-  constexpr bool kTwo = TM == 256 && PRE;  // two barriers a step (below)
-  constexpr int AH = kTwo ? AI / 2 : AI;
-  constexpr int kFirst = BI + 2 + AH;  // kTwo: the loads of a stage that go out first: B, the scales, A's first half
+  constexpr int AH = TWO ? AI / 2 : AI;
+  constexpr int kFirst = BI + 2 + AH;  // TWO: the loads of a stage that go out first: B, the scales, A's first half
   constexpr int kStageA = TM * 128, kStageB = TN * 128, kScaleA = TM * 8, kScaleB = TN * 8;
   __shared__ __attribute__((aligned(1024))) uint8_t sA[S * kStageA];
   __shared__ __attribute__((aligned(1024))) uint8_t sB[S * kStageB];
-  __shared__ __attribute__((aligned(16))) uint8_t sSA[(S + kTwo) * kScaleA];
-  __shared__ __attribute__((aligned(16))) uint8_t sSB[(S + kTwo) * kScaleB];
+  __shared__ __attribute__((aligned(16))) uint8_t sSA[(S + TWO) * kScaleA];
+  __shared__ __attribute__((aligned(16))) uint8_t sSB[(S + TWO) * kScaleB];
   __shared__ __attribute__((aligned(16))) uint32_t sDummy[8 * 64];
   __shared__ unsigned arrive_slot;
 
@@ -699,14 +701,14 @@ __global__ __launch_bounds__(512) void gemm4_lds_kernel(Gemm4Args p) {
   const i32x4 brs = make_rsrc_words(p.b + b_base, clamp_bytes(b_total - b_base));
   const int lr = lane >> 3, lp = lane & 7;
   const int c = lp ^ lr;
-  // A in slabs of 8 rows, AI per wave. kTwo: in two halves, half h the h-th half of the rows of each of the
+  // A in slabs of 8 rows, AI per wave. TWO: in two halves, half h the h-th half of the rows of each of the
   // tile's two wave rows, dealt to the waves in turn.
   uint32_t a_off[AI], b_off[BI];
   int a_slab[AI];
 #pragma unroll
   for (int j = 0; j < AI; ++j) {
     const int i = (j % AH) * 8 + w;
-    a_slab[j] = kTwo ? (i / (TM / 32)) * (TM / 16) + (j / AH) * (TM / 32) + i % (TM / 32) : w * AI + j;
+    a_slab[j] = TWO ? (i / (TM / 32)) * (TM / 16) + (j / AH) * (TM / 32) + i % (TM / 32) : w * AI + j;
     const int r = a_slab[j] * 8 + lr;
     a_off[j] = m0 + r < p.m ? (uint32_t)(r * p.lda + c * 16) : kOobOffset;
   }
@@ -738,7 +740,7 @@ __global__ __launch_bounds__(512) void gemm4_lds_kernel(Gemm4Args p) {
     sb_off = sb_wave && rb < p.n ? (uint32_t)((int64_t)rb * p.lds_b + (lane & 1) * 4) : kOobOffset;
     sa_step = sb_step = 8;
   }
-  const uint32_t lds_a = lds_addr(&sA[kTwo ? 0 : w * (TM / 8) * 128]), lds_b = lds_addr(&sB[w * (TN / 8) * 128]);
+  const uint32_t lds_a = lds_addr(&sA[TWO ? 0 : w * (TM / 8) * 128]), lds_b = lds_addr(&sB[w * (TN / 8) * 128]);
   const uint32_t lds_sa = sa_wave ? lds_addr(&sSA[w * 256]) : lds_addr(&sDummy[w * 64]);
   const uint32_t lds_sb = sb_wave ? lds_addr(&sSB[w * 256]) : lds_addr(&sDummy[w * 64]);
   const uint32_t lds_sa_step = sa_wave ? kScaleA : 0, lds_sb_step = sb_wave ? kScaleB : 0;
@@ -802,7 +804,7 @@ __global__ __launch_bounds__(512) void gemm4_lds_kernel(Gemm4Args p) {
     }
   };
 
-  if constexpr (kTwo) {
+  if constexpr (TWO) {
     // Two barriers a step, so that loads go out 1.5 steps before they are needed although LDS holds two
     // stages. The step's B fragments are in registers when it begins, its A fragments stream one row of
     // tiles ahead, and stage ks + S follows stage ks into its slot in two parts: B, the scales (in a slot
@@ -814,9 +816,12 @@ __global__ __launch_bounds__(512) void gemm4_lds_kernel(Gemm4Args p) {
     // at 4096 x 8192 x 8192 loads and fragment reads without MFMAs took 131 us of the 145, and take 109 of
     // 139 so. What is left is mostly the matrix cores at the clock the chip holds under them: MFMAs alone
     // take 96. Before -> now, us: 512 x 10240 x 8192 43.3 -> 38.5, 4096 x 10240 x 8192 194.3 -> 189.9,
-    // 4096 x 57344 x 8192 980 -> 944. Tiles of 128 rows lose (64 x 8192 x 28672 34.2 -> 34.9, 200 x 4096 x
-    // 4096 13.6 -> 14.6: half the MFMAs behind each barrier), and so do row-major weights (512 x 10240 x 8192
-    // 53.3 -> 55.1), so those keep the one barrier.
+    // 4096 x 57344 x 8192 980 -> 944 (256x128 tiles in the first). A longer prologue and epilogue pay for it:
+    // on short K the one barrier wins (1000 x 7168 x 2048 15.0 against 15.4, 3000 x 7168 x 2560 48.5 / 50.2,
+    // 1000 x 57344 x 256 43.9 / 46.3), from 3072 to 3584 it is within 2% either way, and at 4096 no shape of
+    // either tile loses (3000 x 7168 69.9 -> 68.3, 2048 x 4096 27.5 -> 27.2): kTwoMinK. Tiles of 128 rows lose
+    // (64 x 8192 x 28672 34.2 -> 34.9, 200 x 4096 x 4096 13.6 -> 14.6: half the MFMAs behind each barrier), and
+    // so do row-major weights (512 x 10240 x 8192 53.3 -> 55.1), so those keep the one barrier.
     // Load i of stage ks: B, the scales, A's first half, then A's second half. The K offset rides soffset,
     // and a stage past the range goes through a descriptor of no bytes (zeros, no memory traffic).
     auto issue_one = [&](int i, int ks, int st, int sc) {
@@ -1109,7 +1114,8 @@ static void launch_stream4(const Gemm4Args& g, const Stream4Plan& p, hipStream_t
 
 // LDS-kernel plan for m > 32 when k % 256 == 0 (and, for row-major scales, 4-byte aligned scale rows):
 // tile and split count by the FP8 LDS kernel's cost model (per-K-step times per tile shape, rounds of
-// 256 workgroups, only 128x128 tiles split K).
+// 256 workgroups, only 128x128 tiles split K). The step times were fitted to the loop of one barrier a step,
+// and both loops share them.
 struct Lds4Plan {
   int tm, tn, tiles, splits, ks_per_split;
 };
@@ -1161,7 +1167,12 @@ static bool lds4_ok(int64_t m, int64_t k, int scale_layout, int64_t lds_a, int64
 template <int TM, int TN, bool PRE, bool SSHUF>
 static void launch_lds4_t(const Gemm4Args& g, const Lds4Plan& p, hipStream_t s) {
   constexpr int S = TM + TN == 512 ? 2 : (TM + TN == 384 ? 3 : 4);
-  hipLaunchKernelGGL((gemm4_lds_kernel<TM, TN, S, PRE, SSHUF>), dim3((unsigned)(p.tiles * p.splits)), dim3(512), 0, s, g);
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(p.tiles * p.splits)), dim3(512), 0, s, g);
+  };
+  if constexpr (TM == 256 && PRE)
+    if (g.k >= kTwoMinK) return go(gemm4_lds_kernel<TM, TN, S, PRE, SSHUF, true>);
+  go(gemm4_lds_kernel<TM, TN, S, PRE, SSHUF, false>);
 }
 
 template <bool PRE, bool SSHUF>
@@ -1189,6 +1200,16 @@ extern "C" int aklr_gemm_a4w4_mxfp4_kernel(int64_t m, int64_t n, int64_t k, int 
   if (b_layout != AKLR_B_PRESHUFFLE_16x16 || scale_layout != AKLR_SCALES_SHUFFLED) return 0;
   const Decode4 d = plan_decode4(m, n, k);
   return d == Decode4::kSkinny || d == Decode4::kSkinny8 ? 0 : 1;
+}
+
+extern "C" int aklr_gemm_a4w4_mxfp4_tile(int64_t m, int64_t n, int64_t k, int b_layout, int* rows, int* cols,
+                                         int* barriers) {
+  if (m <= kDecode4MaxM || n <= 0 || k < 256 || k % 256 != 0) return 0;
+  const Lds4Plan p = plan_lds4(m, n, k);
+  *rows = p.tm;
+  *cols = p.tn;
+  *barriers = p.tm == 256 && b_layout == AKLR_B_PRESHUFFLE_16x16 && k >= kTwoMinK ? 2 : 1;
+  return 1;
 }
 
 extern "C" size_t aklr_gemm_a4w4_mxfp4_workspace_bytes(int64_t m, int64_t n, int64_t k) {

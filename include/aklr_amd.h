@@ -196,6 +196,9 @@ size_t aklr_gemm_a4w4_mxfp4_workspace_bytes(int64_t m, int64_t n, int64_t k);
 /* Which kernel a call of these sizes runs: 0 skinny, 1 stream, 2 tiled (LDS; scales as the library's layouts
  * align them). */
 int aklr_gemm_a4w4_mxfp4_kernel(int64_t m, int64_t n, int64_t k, int b_layout, int scale_layout);
+/* The tile rows and columns of the LDS kernel for such a call and its barriers a K step; 0 (and nothing
+ * written) where that kernel does not run (m <= 32, k % 256 != 0). */
+int aklr_gemm_a4w4_mxfp4_tile(int64_t m, int64_t n, int64_t k, int b_layout, int* rows, int* cols, int* barriers);
 int aklr_gemm_a4w4_mxfp4(const uint8_t* a, int64_t lda, const uint8_t* b, int64_t ldb, const uint8_t* a_scale,
                          int64_t lds_a, const uint8_t* b_scale, int64_t lds_b, const float* bias, void* out,
                          int64_t ldo, int64_t m, int64_t n, int64_t k, int b_layout, int scale_layout,
