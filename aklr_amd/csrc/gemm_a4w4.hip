@@ -1014,31 +1014,45 @@ static Skinny4Plan plan_skinny4(int64_t m, int64_t n, int64_t k) {
 }
 
 // Decode plan of preshuffled weights (m <= 16), where the skinny plan above does not do: its waves each read
-// A and its scales again, and with 2 K steps in flight a CU holds about 20 KB of weights under way.
-// * K <= 8192, 224 to 1792 column tiles (n = 3584 to 28672): the stream kernel at one row tile, one column
-//   tile a wave, an 8-deep weight ring behind 8 A stages, no K split; one compute wave a workgroup up to 640
-//   tiles (n = 10240), two past that, so that the workgroups stay small and many. us, skinny -> this, m = 1 /
-//   8 / 16: 10240 x 8192 11.8 / 12.2 / 13.6 -> 11.4 / 11.6 / 12.3, 8192 x 8192 10.3 / 11.1 / 11.3 -> 9.9 /
-//   10.2 / 10.4, 4096 x 4096 6.05 / 6.48 / 6.6 -> 5.35 / 5.51 / 5.46, 7168 x 2048 4.59 / 4.84 / 5.16 -> 4.52 /
-//   4.55 / 4.70, 3584 x 448 3.25 / 3.38 / 3.41 -> 2.73 / 2.75 / 2.80, 16384 x 4096 9.6 / 9.9 / 10.5 -> 9.6 /
-//   9.8 / 9.9, 28672 x 8192 25.4 / 26.0 / 28.3 -> 25.4 / 25.3 / 26.6.
-// * wider n, m > 8, K = 4096 to 8192: 224-column workgroups (7 waves of two tiles, a 4-deep ring): 57344 x
-//   8192 at m = 16 47.1 -> 43.5 (at 8 43.2 -> 43.6). Shorter K loses (32768 x 2048 at 16 10.8 -> 11.4).
-// * K > 16384, 112 or more groups of 32 columns: the skinny kernel with 8 waves on the workgroup's K range,
-//   two K splits up to 128 groups: 4096 x 28672 at m = 1 / 8 / 16 18.8 / 19.6 / 20.3 -> 14.9 / 14.9 / 16.0,
-//   8192 x 28672 at 8 / 16 26.5 / 31.9 -> 24.2 / 26.1, 16384 x 28672 48.3 / 67.3 -> 43.9 / 49.5. Past 128
-//   groups one row is even (8192 x 28672 23.3 -> 23.5), and keeps its plan, as does K = 16384 (4608 x 16384
-//   at m = 1 11.9 -> 12.2).
+// A and its scales again, and with 2 K steps in flight a CU holds about 20 KB of weights under way. What
+// decides past that is how evenly the workgroups fill the 256 CUs. us, skinny -> this, cold weights:
+// * K <= 8192, 224 to 768 column tiles (n = 3584 to 12288), the stream kernel with one compute wave (one column
+//   tile) a workgroup, an 8-deep weight ring behind 8 A stages, no K split, up to three workgroups a CU: m = 8,
+//   4096 x 4096 6.5 -> 5.5, 10240 x 2048 5.7 -> 5.4, 10240 x 7680 15% less, 12288 x 4096 8.6 -> 8.3; past 768
+//   tiles it loses (13312 x 4096 8.7 -> 9.1). The skinny waves' K ranges come out even only near K = 8192, where
+//   the gain is small (8192 x 8192 10.8 -> 10.5) and a part-filled round eats it: past K = 7936 it runs up to
+//   304 tiles, at 481 to 512, and past 512 from 8 rows (10240 x 8192 at m = 8 / 16 12.1 -> 12.1 / 13.6 -> 12.8;
+//   at m = 1 11.6 -> 11.8, 9216 x 8192 3.7% more; 6144 x 8192 at m = 16 4% more).
+// * K = 4096 to 8192, m >= 12, two compute waves a workgroup (32 columns), where those make 385 to 512 workgroups
+//   or 769 to 896: 16384 x 8192 at 16 16.4 -> 15.3, 28672 x 8192 27.5 -> 25.3, 14336 x 4096 9.5 -> 9.3; at m = 1
+//   up to 4% more. With 513 to 640 workgroups m = 12 is up to 2% either way and m = 1 12% more, with 736 to 768
+//   all lose (24576 x 8192 at 16 23.1 -> 23.9), and so does K = 2048 (28672 at 16 10.0 -> 10.2).
+// * wider n, K = 4096 to 8192, m >= 12, 224-column workgroups (7 waves of two tiles, a 4-deep ring), where they
+//   fill the last round of CUs to 15/16: 57344 x 8192 (256) at m = 12 / 16 45.8 -> 43.9 / 48.0 -> 44.3, 114688 x
+//   8192 (512) at 16 94.1 -> 86.3. At m = 9 it takes up to 5% more, and with a part-filled round up to 40%
+//   (28688 x 8192, 129 workgroups, at 16 28.2 -> 36.3; 65536 x 8192, 293, 54.8 -> 72.2). Shorter K loses
+//   (32768 x 2048 at 16 10.8 -> 11.4).
+// * K > 16384, the skinny kernel with 8 waves on the workgroup's K range: 112 to 128 groups of 32 columns in two
+//   K splits (4096 x 28672 at m = 1 / 8 / 16 18.7 -> 14.8 / 19.2 -> 15.4 / 19.9 -> 16.7; K = 16384 keeps its plan,
+//   4608 x 16384 at m = 1 11.8 -> 12.5); from 132 groups, 8 rows and K = 18432 on without a split (8192 x 28672 at
+//   m = 8 / 16 26.2 -> 24.9 / 35.0 -> 27.4, at m = 2 23.3 -> 24.6; 18432 x 16448 at m = 9 6% more), but not with 257 to
+//   415 groups, between one workgroup a CU and 1.6 (9216 x 28672 at m = 8 7.7% more, 12288 x 28672 at 12 2.1%).
 enum class Decode4 { kSkinny, kStream1, kStream2, kStream14, kSkinny8 };
 static Decode4 plan_decode4(int64_t m, int64_t n, int64_t k) {
-  const int64_t tiles = (n + 15) / 16;
+  const int64_t tiles = (n + 15) / 16, groups = (n + 31) / 32;
   if (k <= 8192) {
-    if (tiles >= 224 && tiles <= 1792) return tiles <= 640 ? Decode4::kStream1 : Decode4::kStream2;
-    if (tiles > 1792 && m > 8 && k >= 4096) return Decode4::kStream14;
-  } else if (k > 16384 && n >= 112 * 32 && (m > 1 || n <= 128 * 32)) {
-    return Decode4::kSkinny8;
+    if (tiles >= 224 && tiles <= 768) {
+      const bool even = tiles <= 304 || (tiles > 480 && tiles <= 512) || (tiles > 512 && m >= 8);
+      return k <= 7936 || even ? Decode4::kStream1 : Decode4::kSkinny;
+    }
+    if (tiles < 224 || k < 4096 || m < 12) return Decode4::kSkinny;
+    if (tiles <= 1792) return groups <= 512 || groups > 768 ? Decode4::kStream2 : Decode4::kSkinny;
+    const int64_t last = (n + 223) / 224 % 256;
+    return last == 0 || last >= 240 ? Decode4::kStream14 : Decode4::kSkinny;
   }
-  return Decode4::kSkinny;
+  if (k <= 16384 || n < 112 * 32) return Decode4::kSkinny;
+  if (groups <= 128) return Decode4::kSkinny8;
+  return m >= 8 && k >= 18432 && groups >= 132 && (groups <= 256 || groups >= 416) ? Decode4::kSkinny8 : Decode4::kSkinny;
 }
 static Skinny4Plan plan_skinny8(int64_t n, int64_t k) {
   Skinny4Plan p;
