@@ -176,9 +176,12 @@ def api(contract_id: str, run_fn, native: str | None = None):
     launches and returns the outputs. The result is the api function, with ``.serving`` and
     ``.fallback_reason`` of the same signature attached. ``native`` names the op's function in
     ``aklr_amd._host``: a call on GPU tensors goes there first, and comes back here (``.general``) where that
-    function leaves the decision to the plan. A call whose first argument is not on a GPU skips it, so the
-    ops answer without the native library there, as before."""
+    function leaves the decision to the plan. The function is loaded by the op's first call whose first
+    positional argument is a GPU tensor; until then calls go to the plan, so the ops answer without the
+    native library where they need none."""
     import functools
+
+    import torch
 
     from . import _lib
 
@@ -221,7 +224,9 @@ def api(contract_id: str, run_fn, native: str | None = None):
             def call(*args, **kwargs):
                 nonlocal host
                 if host is None:
-                    if not (args and getattr(args[0], "is_cuda", False)) or disabled(contract_id):
+                    # what is no tensor (a tracer's stand-in) is asked nothing: the plan refuses it without raising
+                    x = args[0] if args else None
+                    if not isinstance(x, torch.Tensor) or x.is_cuda is not True or disabled(contract_id):
                         return general(*args, **kwargs)
                     host = _lib.host_function(native)
                     if host is None:

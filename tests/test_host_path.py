@@ -40,6 +40,22 @@ def test_cpu_calls_are_left_to_the_general_path(native_lib, name):
         op(x, nope=1)
 
 
+class _Untouchable:
+    def __getattr__(self, name):
+        raise RuntimeError(f"{name} was asked for")
+
+
+@pytest.mark.parametrize("name", sorted(NATIVE))
+@pytest.mark.parametrize("kind", ["proxy", "untouchable"])
+def test_what_is_no_tensor_is_refused_without_raising(name, kind):
+    """A tracer's stand-in, or any object, answers no question that the plan would not ask."""
+    graph = torch.fx.Graph()
+    x = torch.fx.Proxy(graph.placeholder("x"), torch.fx.Tracer()) if kind == "proxy" else _Untouchable()
+    count = {"quant_gemm_fp8": 3}.get(name, 1 if name.startswith("quant_") else 4)
+    assert NATIVE[name](*(x,) * count) is FallbackReason.OUT_OF_CONTRACT
+    assert NATIVE[name].serving(*(x,) * count) is FallbackReason.OUT_OF_CONTRACT
+
+
 def _same(a, b):
     if isinstance(a, tuple):
         return isinstance(b, tuple) and len(a) == len(b) and all(_same(x, y) for x, y in zip(a, b))
