@@ -3,9 +3,10 @@
 In-tree build for gfx950 only: every ``.hip`` file compiles to an object in ``aklr_amd/_build/`` (in
 parallel), then hipcc links them into one shared library exporting the C ABI of
 ``include/aklr_amd.h``. Mirrors the role of aklr/core/jit/hip_extension.py (hipcc, ``-O3``, one arch),
-without torch in the loop: the library has no torch types in its interface. ``aklr_amd/_host.so``
+without torch in the loop: the library has no torch types in its interface. ``aklr_amd/_host.*.so``
 (``csrc/host/host.cpp``) is the one part that has them: the ops' host work as a Python extension, built
-with the host compiler against torch's headers and linked to the library beside it.
+with the host compiler against torch's headers and linked to the library beside it. It refuses another
+torch version than the one it was built with.
 """
 from __future__ import annotations
 
@@ -13,6 +14,7 @@ import concurrent.futures
 import os
 import shutil
 import subprocess
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -20,7 +22,7 @@ CSRC = PKG / "csrc"
 BUILD_DIR = PKG / "_build"
 LIB_PATH = PKG / "libaklr_amd.so"
 HOST_SRC = CSRC / "host" / "host.cpp"
-HOST_PATH = PKG / "_host.so"
+HOST_PATH = PKG / f"_host{sysconfig.get_config_var('EXT_SUFFIX')}"  # no other Python imports it
 ARCH = "gfx950"
 
 # Packed-fp32 VALU ops are switched off: the kernels' fp32 arithmetic stays scalar per lane. The sources
@@ -55,9 +57,7 @@ def _compile(src: Path) -> Path:
 
 
 def _link_host() -> None:
-    """``_host.so``: found beside ``libaklr_amd.so`` by its run path, torch's libraries by the process."""
-    import sysconfig
-
+    """``_host.*.so``: it finds ``libaklr_amd.so`` by its run path, torch's libraries by the process."""
     import torch
 
     root = Path(torch.__file__).resolve().parent
@@ -67,7 +67,7 @@ def _link_host() -> None:
     tmp = HOST_PATH.with_suffix(".so.tmp")
     cmd = [
         os.environ.get("CXX") or "g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1",
-        "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{root}/include",
+        "-DUSE_ROCM=1", f'-DAKLR_TORCH_VERSION="{torch.__version__}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{root}/include",
         f"-I{root}/include/torch/csrc/api/include", f"-I{rocm}/include", f"-I{sysconfig.get_paths()['include']}",
         str(HOST_SRC), "-o", str(tmp), f"-L{root}/lib", "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-ltorch",
         "-lc10_hip", "-lc10", f"-L{PKG}", f"-l:{LIB_PATH.name}", "-Wl,-rpath,$ORIGIN",
@@ -79,7 +79,7 @@ def _link_host() -> None:
 
 
 def build(verbose: bool = False) -> Path:
-    """Compile every kernel source, link ``libaklr_amd.so`` and build ``_host.so`` on it; returns the
+    """Compile every kernel source, link ``libaklr_amd.so`` and build ``_host.*.so`` on it; returns the
     library's path."""
     BUILD_DIR.mkdir(exist_ok=True)
     srcs = sources()

@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes
 import hashlib
 import threading
+import warnings
 from pathlib import Path
 
 from ._build import LIB_PATH
@@ -91,6 +92,7 @@ class NativeLibraryError(RuntimeError):
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
 _digest: str | None = None
+_host_missing = False  # aklr_amd._host did not load: not tried again
 
 
 def lib() -> ctypes.CDLL:
@@ -121,15 +123,23 @@ def lib() -> ctypes.CDLL:
 def host_function(name: str):
     """The native host path of an op (``aklr_amd._host``): called with a call's args tuple and kwargs dict,
     it returns the outputs or None for a call the general path has to decide. None when the library itself
-    is not built (the general path says so where it needs it)."""
-    if not Path(LIB_PATH).exists():
+    is not built or does not load (the general path says so where it needs it), and when only ``_host`` does
+    not: it is tied to one Python and one torch, and without it the same kernels are called from Python, in
+    about 10 us more a call; a warning says so once."""
+    global _host_missing
+    if _host_missing or not Path(LIB_PATH).exists():
         return None
-    lib()  # checks its ABI version
+    try:
+        lib()  # checks its ABI version
+    except (NativeLibraryError, OSError):
+        return None
     try:
         from . import _host
     except ImportError as e:
-        raise NativeLibraryError(f"aklr_amd._host is not built or does not load: run "
-                                 f"`python -c 'import __graft_entry__ as g; g.build()'` ({e})") from e
+        _host_missing = True
+        warnings.warn(f"aklr_amd._host is not built for this Python and torch, calls take the slower host path: run "
+                      f"`python -c 'import __graft_entry__ as g; g.build()'` ({e})", RuntimeWarning, stacklevel=3)
+        return None
     return getattr(_host, name)
 
 

@@ -78,7 +78,11 @@ const at::Tensor* plain(PyObject* o) {
 
 bool is_true_attr(PyObject* o, PyObject* name, bool* out) {
   PyObject* v = nullptr;
-  if (_PyObject_LookupAttr(o, name, &v) < 0) return false;
+#if PY_VERSION_HEX >= 0x030D0000
+  if (PyObject_GetOptionalAttr(o, name, &v) < 0) return false;
+#else
+  if (_PyObject_LookupAttr(o, name, &v) < 0) return false;  // the same function before it was public
+#endif
   *out = v == Py_True;
   Py_XDECREF(v);
   return true;
@@ -376,7 +380,20 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", "the ops' per-call host w
 
 }  // namespace
 
+// The checks above read torch's own objects, whose layout belongs to one version.
+static bool same_torch() {
+  PyObject* torch = PyImport_ImportModule("torch");
+  PyObject* version = torch ? PyObject_GetAttrString(torch, "__version__") : nullptr;
+  Py_XDECREF(torch);
+  if (!version) return false;
+  const bool same = PyUnicode_Check(version) && PyUnicode_CompareWithASCIIString(version, AKLR_TORCH_VERSION) == 0;
+  if (!same) PyErr_Format(PyExc_ImportError, "built with torch %s, not %S", AKLR_TORCH_VERSION, version);
+  Py_DECREF(version);
+  return same;
+}
+
 PyMODINIT_FUNC PyInit__host() {
+  if (!same_torch()) return nullptr;
   if (aklr_abi_version() != 1) {
     PyErr_SetString(PyExc_ImportError, "libaklr_amd.so ABI version does not match aklr_amd._host");
     return nullptr;

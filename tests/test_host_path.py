@@ -9,11 +9,15 @@ not take, it returns None and the op's answer is the general path's (outputs or 
 """
 from __future__ import annotations
 
+import importlib.util
+import sys
+import warnings
+
 import pytest
 import torch
 
 import aklr_amd
-from aklr_amd import _lib, layouts, workloads
+from aklr_amd import _build, _lib, layouts, workloads
 from aklr_amd.dispatch import FallbackReason
 from tests.helpers import say
 
@@ -54,6 +58,41 @@ def test_what_is_no_tensor_is_refused_without_raising(name, kind):
     count = {"quant_gemm_fp8": 3}.get(name, 1 if name.startswith("quant_") else 4)
     assert NATIVE[name](*(x,) * count) is FallbackReason.OUT_OF_CONTRACT
     assert NATIVE[name].serving(*(x,) * count) is FallbackReason.OUT_OF_CONTRACT
+
+
+def _not_loading(monkeypatch):
+    monkeypatch.delattr(aklr_amd, "_host", raising=False)
+    monkeypatch.setitem(sys.modules, "aklr_amd._host", None)
+    monkeypatch.setattr(_lib, "_host_missing", False)
+
+
+def test_an_extension_that_does_not_load_leaves_the_general_path(native_lib, monkeypatch):
+    _not_loading(monkeypatch)
+    with pytest.warns(RuntimeWarning, match="_host"):
+        assert _lib.host_function("quant_fp8") is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")  # once
+        assert _lib.host_function("gemm_fp8") is None
+
+
+def test_the_extension_refuses_another_torch(native_lib, monkeypatch):
+    spec = importlib.util.spec_from_file_location("another._host", _build.HOST_PATH)
+    monkeypatch.setattr(torch, "__version__", "1.0.0")
+    with pytest.raises(ImportError, match="built with torch"):
+        importlib.util.module_from_spec(spec)
+
+
+@pytest.mark.gpu
+def test_ops_serve_without_the_extension(monkeypatch):
+    say("host path without the extension")
+    from aklr_amd import quant
+
+    _not_loading(monkeypatch)
+    op = quant.api("per_group_quant_fp8@1.0", quant._run_fp8, native="quant_fp8")(quant.per_group_quant_fp8.__wrapped__)
+    x = workloads.activations(5, 1024, seed=5, device=DEV)
+    with pytest.warns(RuntimeWarning, match="_host"):
+        got = op(x)
+    assert _same(got, quant.per_group_quant_fp8.general(x)) and op(x.float()) is FallbackReason.OUT_OF_CONTRACT
 
 
 def _same(a, b):
