@@ -7,12 +7,11 @@
 // accumulates straight into the fp32 result.
 //
 // * skinny (m <= 16 but for the stream plans of preshuffled weights, plan_decode4, and 16 < m <= 32 with
-//   unaligned row-major scales): weight streaming -- a
-//   workgroup owns 32 columns and a K range, each wave a contiguous K sub-range with a register ring;
-//   fixed-order wave reduction in LDS, then (when K is also split across workgroups) fp32 partials
-//   summed in split order by the last workgroup to arrive.
-// * stream (16 < m <= 32, and m <= 16 by plan_decode4): the FP8 stream kernel's design -- compute waves stream their own weight
-//   columns into register rings while a loader wave stages A and its scales in LDS for all of them.
+//   unaligned row-major scales): weight streaming -- a workgroup owns 32 columns and a K range, each wave a
+//   contiguous K sub-range with a register ring; fixed-order wave reduction in LDS, then (when K is also split
+//   across workgroups) fp32 partials summed in split order by the last workgroup to arrive.
+// * stream (16 < m <= 32, and m <= 16 by plan_decode4): the FP8 stream kernel's design -- compute waves stream
+//   their own weight columns into register rings while a loader wave stages A and its scales in LDS for all.
 // * lds (m > 32, k % 256 == 0): the FP8 LDS kernel's tiles and direct-to-LDS ring, K steps of 256
 //   values with the scale bytes staged beside the codes (see gemm4_lds_kernel).
 // * tile (m > 32, other k): 128x128 tiles, 4 waves of 64x64, K steps of 256 (128 bytes per row)
@@ -245,14 +244,14 @@ __global__ __launch_bounds__(NW * 64) void gemm4_skinny_kernel(Gemm4Args p) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// stream (16 < m <= 32): the FP8 stream kernel's design (gemm_a8w8.hip) on e2m1. A workgroup owns
+// stream (16 < m <= 32, and m <= 16 on preshuffled weights by plan_decode4): the FP8 stream kernel's design
+// (gemm_a8w8.hip) on e2m1. A workgroup owns
 // NW * NT * 16 output columns and a K range of 256-value blocks (128 bytes of codes per row). Its NW
 // compute waves stream their NT weight tiles from HBM straight into a D-deep register ring (codes and
 // the tiles' e8m0 scales); one loader wave moves each K block of A -- the codes as whole 128-byte rows
 // (row r of row tile mt at mt * 2048 + r * 128, its 16-byte chunk c at position c ^ (r & 7), so the
 // fragment reads are conflict-free) and the rows' 8 scale bytes, 256 bytes per 32 rows in the
-// caller's layout -- into an
-// NS-stage LDS ring. One LDS-fenced barrier per block hands a stage over; the MFMA applies both
+// caller's layout -- into an NS-stage LDS ring. One LDS-fenced barrier per block hands a stage over; the MFMA applies both
 // scales, so there is no fold. Lane groups past k load zero codes and take scale 1.0, so padding scale
 // bytes never reach the MFMA. Row-major scales need 4-byte-aligned rows (stream4_ok).
 template <int NT>
@@ -987,7 +986,7 @@ __global__ __launch_bounds__(512) void gemm4_lds_kernel(Gemm4Args p) {
 // ---------------------------------------------------------------------------------------------
 static constexpr int64_t kDecode4MaxM = 32;
 
-// Skinny plan (m <= 32), measured on MI355X over the Llama-70B MXFP4 shapes at m = 1 and 32: one or
+// Skinny plan (m <= 32; plan_decode4 says where others replace it), measured on MI355X over the Llama-70B MXFP4 shapes at m = 1 and 32: one or
 // two 16-row tiles, two 16-column tiles and 4 waves per workgroup, 2 K steps in flight per wave
 // (best or within 3% of the best of 2-8 in flight, 4 or 8 waves, 1-4 column tiles and 1-4 K splits);
 // K is split in two only when the columns give fewer than 512 waves (small n).

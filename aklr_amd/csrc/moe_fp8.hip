@@ -554,7 +554,15 @@ __device__ __forceinline__ float round_bf16(float v) { return __uint_as_float(f3
 // direct-to-LDS ring of as many stages as LDS holds (3 for TM <= 128, 2 for 256), with the swizzled
 // LDS tiles, load schedule and fold of the dense LDS kernel. GATEUP orders the tile's 256 weight rows
 // as (gate 16, up 16) pairs over 128 intermediate columns, so tiles nt = 2q and 2q + 1 of a wave are
-// the gate and the up of the same 16 columns. LDS comes from the caller's buffer (moe_smem_bytes).
+// the gate and the up of the same 16 columns. LDS comes from the caller's buffer, as MoeSmem lays it out.
+//
+// DOWN items of the 64- and 128-row classes take `tiles` consecutive weight tiles from pn on, in one stream of
+// tiles * KB steps through the ring (the 256-row class, whose accumulators leave no registers for it, one): a
+// tile's results are stored between two steps while the next tile's stages are in flight. On short K an item of
+// one tile is mostly its own start (a ticket, the block's entry, the b_scale rows and the first stages, one after
+// the other): 128 tokens on 256 experts of 7168 x 256 (2 K blocks, 28 tiles) took 100 us for 460 MB of weights,
+// and 75 in items of 6 tiles. From 16 K blocks on items keep one tile (32 steps an item instead of 16: 4096
+// tokens at 2048, 3420 -> 3470 us a call, the last items end too far apart).
 template <int TM>
 struct MoeSmem {
   static constexpr int S = TM == 256 ? 2 : 3, MT = TM / 32;
@@ -568,13 +576,6 @@ constexpr int kMoeSmemBytes =
         : (MoeSmem<128>::kBytes > MoeSmem<64>::kBytes ? MoeSmem<128>::kBytes : MoeSmem<64>::kBytes);
 static_assert(kMoeSmemBytes <= 160 * 1024, "LDS");
 
-//
-// DOWN items of the 64- and 128-row classes take `tiles` consecutive weight tiles from pn on, in one stream of
-// tiles * KB steps through the ring (the 256-row class, whose accumulators leave no registers for it, one): a tile's results are stored between two steps while the next tile's stages are in flight. On short
-// K an item of one tile is mostly its own start (a ticket, the block's entry, the b_scale rows and the first
-// stages, one after the other): 128 tokens on 256 experts of 7168 x 256 (2 K blocks, 28 tiles) took 100 us
-// for 460 MB of weights, and 75 in items of 6 tiles. From 16 K blocks on items keep one tile (32 steps an
-// item instead of 16: 4096 tokens at 2048, 3420 -> 3470 us a call, the last items end too far apart).
 template <int MODE, bool PRE, int TM>
 __device__ __forceinline__ void moe_item(const MoeGemmArgs& p, uint8_t* smem, int cls, int blk, int pn, int tiles) {
   using L = MoeSmem<TM>;
